@@ -396,6 +396,80 @@ int sumpyhip_m2l_apply_noalloc(int precision, int nlevels, const sumpyhip_m2l_le
                                int nl, int nm, int npad, int kpad, const int *off_t,
                                const int *off_s, int ncirc, void *stream);
 
+/* {{{ M2L folded by reflection symmetry (whole traversals of an octree)
+ *
+ * Replaces M2LPreprocessMultipole / M2LUsingTranslationClassesDependentData /
+ * M2LPostprocessLocal over all levels of one order (sumpy/fmm.py:777-920) for
+ * class vectors n h with integer |n_i| <= 3 and PDE-compressed expansions of
+ * orders 1..12, precision 0 (FP64) or 1 (FP32); complex kernels hold (re, im).
+ * A vector n has the code (n_x + 3) 49 + (n_y + 3) 7 + n_z + 3. */
+
+/* out[41]: folded axes ax, row blocks, k pairs, row blocks [8] and k pairs [8]
+ * by parity class; of the class data's layout in FP32 and in FP64: strides S0,
+ * S1 and entries [3], then the first entry of every parity class [8] of each. */
+int sumpyhip_m2l_fold_sizes(int order, int *out);
+
+/* Workgroups of sumpyhip_m2l_fold_apply that the current GPU holds at once. */
+int sumpyhip_m2l_fold_max_wg(int precision, int is_complex, int order, int *out);
+
+/* keys[i] = 8 * (plan level) + octant of target box i, 8 * nlev for a box
+ * without list-2 sources or of a level outside the plan; lev_slot[nlevels]
+ * (host): plan level of a tree level, -1 outside; block_base[nlev + 1] (host):
+ * first block of each plan level. */
+int sumpyhip_m2l_fold_keys(int ax, int nlevels, const int *lev_slot, int nlev,
+                           const int *block_base, double root_extent, int nboxes,
+                           const int *box_levels, const double *centers, int ntgt,
+                           const int *target_boxes, const int *starts, int *keys,
+                           void *stream);
+
+/* The plan: from the sorted keys, their permutation and the first position of
+ * each key, the target of every (tile, column) (tile_target, preset to -1; 4
+ * tiles of 16 columns per block), the source of every (tile, vector, column)
+ * (src, 343 x 16 per tile, preset to -1), the tiles of a block with a canonical
+ * vector (present, 343 per block, preset to 0), and per block the slots
+ * (maxslots each, by type: the set of folded axes without a component), the cost
+ * before each of them, the slots up to each type (type_end, 8 per block) and
+ * the block's cost.  class_code: code of every translation class. */
+int sumpyhip_m2l_fold_plan(int ax, int nlevels, const int *lev_slot, int nlev,
+                           const int *block_base, double root_extent, int nboxes,
+                           const int *box_levels, const double *centers, int ntgt,
+                           const int *target_boxes, const int *starts, const int *lists,
+                           const int *classes, const int *class_code,
+                           const int *sorted_keys, const long long *order,
+                           const long long *key_start, int *tile_target, int *tgt_pos,
+                           int *src, int *present, int maxslots, int *slots,
+                           int *slot_costs, int *type_end, long long *block_costs,
+                           void *stream);
+
+/* One level's class data of the canonical vectors, ntable of them, from the
+ * class data (circulant shape circ_shape): rep[ntable] the class of a vector
+ * (-1: none), sgn[ntable] the reflection between the two. */
+int sumpyhip_m2l_fold_table(int precision, int is_complex, int order, int ntable,
+                            const int *circ_shape, const int *rep, const int *sgn,
+                            const double *class_data, void *table, void *stream);
+
+/* Multipoles of nboxes boxes in padded k order (kpad entries per box in the
+ * compute precision). */
+int sumpyhip_m2l_fold_pack(int precision, int is_complex, int nboxes, int nstored, int kpad,
+                           const double *src, const int *kmap, void *packed, void *stream);
+
+/* The contraction: overwrites the rows of out (nstored values per box, from box
+ * box0 on) of the plan's targets.  block_level: plan level of every block;
+ * block_cost[nblocks + 1]: exclusive sums of block_costs; level_stride: table
+ * entries per level; partial: 2 max_wg x 4 x planes x row blocks x 256 values;
+ * min_slots: slots a workgroup takes at least.  Deterministic. */
+int sumpyhip_m2l_fold_apply(int precision, int is_complex, int order, int nblocks,
+                            int maxslots, int box0, int nboxes, int nstored,
+                            const int *tile_target, const int *src, const int *slots,
+                            const int *slot_costs, const int *type_end,
+                            const int *block_level, const long long *block_cost,
+                            const int *rowmap, const int *off_t, const int *off_s,
+                            const void *packed, const void *table, long long level_stride,
+                            int max_wg, int min_slots, void *partial, double *out,
+                            void *stream);
+
+/* }}} */
+
 /* Split-BF16 form (precision 2) support, no reference counterpart (a layout
  * of this library's split-BF16 contraction): the class data of nclasses
  * classes (circulant shape circ_shape, as written by sumpyhip_m2l_class_data)

@@ -111,6 +111,14 @@ _SIGNATURES = {
                                   _P],
     "sumpyhip_qbx2d_adjoint": [_I, _I, _I, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _D, _P,
                                _P, _P, _P, _P, _P, _P, _P, _P, _P, _P],
+    "sumpyhip_m2l_fold_sizes": [_I, _P],
+    "sumpyhip_m2l_fold_max_wg": [_I, _I, _I, _P],
+    "sumpyhip_m2l_fold_keys": [_I, _I, _P, _I, _P, _D, _I, _P, _P, _I, _P, _P, _P, _P],
+    "sumpyhip_m2l_fold_plan": [_I, _I, _P, _I, _P, _D, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P,
+                               _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P],
+    "sumpyhip_m2l_fold_table": [_I, _I, _I, _I, _P, _P, _P, _P, _P, _P],
+    "sumpyhip_m2l_fold_pack": [_I, _I, _I, _I, _I, _P, _P, _P, _P],
+    "sumpyhip_m2l_fold_apply": [_I]*8 + [_P]*12 + [_L, _I, _I, _P, _P, _P],
     "sumpyhip_m2l_pack_bf16_class_data": [_I, _P, _I, _I, _I, _P, _P, _P],
     "sumpyhip_m2l_class_data": [_I, _I, _I, _P, _I, _P, _I, _I, _D, _P, _P],
     "sumpyhip_m2l_preprocess": [_I, _I, _I, _P, _I, _P, _P, _P],

@@ -17,9 +17,11 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 
-HIP_SOURCES = ["misc.hip", "p2p.hip", "expansions.hip", "m2l.hip", "octant.hip", "helmholtz.hip",
-               "tree_gpu.hip", "h2d.hip", "qbx.hip",
-               "taylor2d.hip"]
+# (the slowest to compile first)
+HIP_SOURCES = [f"m2l_fold_{name}{orders}.hip" for orders in ("b", "a", "")
+               for name in ("c128", "c64", "f64", "f32")] + [
+    "misc.hip", "p2p.hip", "expansions.hip", "m2l.hip", "m2l_fold.hip", "octant.hip",
+    "helmholtz.hip", "tree_gpu.hip", "h2d.hip", "qbx.hip", "taylor2d.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17",

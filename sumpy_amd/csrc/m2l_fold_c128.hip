@@ -1,0 +1,10 @@
+// complex FP64 kernels of the folded M2L contraction, orders 1 to 8.
+#include "m2l_fold.h"
+
+namespace sumpyhip {
+namespace m2l_fold {
+
+SUMPYHIP_FOLD_INSTANCE(c128, double, true, 1, 8)
+
+}  // namespace m2l_fold
+}  // namespace sumpyhip

@@ -517,16 +517,62 @@ class SumpyExpansionWrangler:
 
     def multipole_to_local(self, actx, level_start_target_box_nrs, target_boxes,
                            src_box_starts, src_box_lists, mpole_exps):
-        """M2L of every level.  With translation classes, each run of
+        """M2L of every level.  On an octree the whole pass is one contraction
+        folded by the kernel's reflection symmetry
+        (:mod:`sumpy_amd.m2l_fold`); otherwise, or where the autotuner
+        measures them to be faster, the class matrices level by level
+        (:meth:`_m2l_class_matrices`).  The result equals the reference's
+        per-level loop (``fmm.py:777-920``)."""
+        from sumpy_amd import m2l_fold
+        args = (actx, _host(level_start_target_box_nrs), target_boxes, src_box_starts,
+                src_box_lists, mpole_exps)
+        folded = m2l_fold.runs(self, *args[1:5])
+        if folded is None or not self._m2l_prefers_folded(folded, args):
+            return self._m2l_class_matrices(*args)
+        return self._m2l_folded(folded, args)
+
+    def _m2l_folded(self, folded, args):
+        from sumpy_amd import m2l_fold
+        actx, mpole_exps = args[0], args[-1]
+        local_exps = self.local_expansion_zeros(actx)
+        for order, levels in folded:
+            m2l_fold.apply(actx, self, order, levels, mpole_exps, local_exps)
+        return local_exps
+
+    def _m2l_prefers_folded(self, folded, args):
+        """Without autotuning: yes.  With it: whether the folded form is the
+        faster one on this wrangler's first pass (3 runs of each, the class
+        matrices with their tuned split), kept for its later passes."""
+        if not self.tree_indep.autotune:
+            return True
+        got = self._memo.get("m2l_prefers_folded")
+        if got is None:
+            if torch.cuda.is_current_stream_capturing():
+                return True  # nothing is timed inside a graph capture
+            times = []
+            for run in (lambda: self._m2l_class_matrices(*args),
+                        lambda: self._m2l_folded(folded, args)):
+                run()  # plans, schedules, the split tuner
+                e0, e1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                e0.record()
+                for _ in range(3):
+                    run()
+                e1.record()
+                e1.synchronize()
+                times.append(e0.elapsed_time(e1))
+            got = self._memo["m2l_prefers_folded"] = times[1] <= times[0]
+        return got
+
+    def _m2l_class_matrices(self, actx, starts, target_boxes, src_box_starts, src_box_lists,
+                            mpole_exps):
+        """M2L by class matrices.  With translation classes, each run of
         consecutive levels of one order is preprocessed in one launch, the
         levels of an order are contracted in a single MFMA launch
         (:func:`sumpy_amd.e2e.m2l_apply_levels`) and each run is
         postprocessed in one launch (source and target of an M2L share the
-        level, so the postprocessing scale ratio is 1 on every level); the
-        result equals the reference's per-level loop (``fmm.py:777-920``)."""
+        level, so the postprocessing scale ratio is 1 on every level)."""
         from sumpy_amd.e2e import TILE, m2l_apply_levels
         local_exps = self.local_expansion_zeros(actx)
-        starts = _host(level_start_target_box_nrs)
         # translations without preprocessing (the 2D Bessel locals) take the
         # classes' data in the per-level M2L operator itself
         use_pre = (self.supports_translation_classes
