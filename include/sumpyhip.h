@@ -172,6 +172,16 @@ int sumpyhip_octant_translate(int ngroups, const int *group_targets,
                               double *tgt_expansions, int tgt_base_ibox, void *partial,
                               void *stream);
 
+/* The same for planes = 2 interleaved planes per coefficient (complex
+ * expansions under real matrices; partial: twice the values) or planes = 1;
+ * at most 256 complex coefficients. */
+int sumpyhip_octant_translate_planes(int planes, int ngroups, const int *group_targets,
+                                     const int *group_inputs, const int *group_octant_mask,
+                                     int nitems, const int *items, int n_out, int n_in,
+                                     const double *T_frag, const double *src_expansions,
+                                     int src_base_ibox, double *tgt_expansions,
+                                     int tgt_base_ibox, void *partial, void *stream);
+
 /* L2P, replaces E2PFromSingleBox.__call__ (sumpy/e2p.py:123-226); overwrites
  * pot (and the gradient when given) for the targets of each box. */
 int sumpyhip_l2p(int kernel_id, const sumpyhip_expn *expn, int ntgt_boxes,

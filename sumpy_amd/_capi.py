@@ -109,6 +109,8 @@ _SIGNATURES = {
     "sumpyhip_m2l_class_data_helmholtz": [_I, _I, _P, _I, _P, _I, _I, _D, _D, _D, _P, _P],
     "sumpyhip_octant_translate": [_I, _P, _P, _P, _I, _P, _I, _I, _P, _P, _I, _P, _I, _P,
                                   _P],
+    "sumpyhip_octant_translate_planes": [_I, _I, _P, _P, _P, _I, _P, _I, _I, _P, _P, _I, _P, _I,
+                                         _P, _P],
     "sumpyhip_qbx2d_adjoint": [_I, _I, _I, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _D, _P,
                                _P, _P, _P, _P, _P, _P, _P, _P, _P, _P],
     "sumpyhip_m2l_fold_sizes": [_I, _P],

@@ -26,6 +26,7 @@ from sumpy_amd.tools import as_i32, expansion_k, helmholtz_k, planes, set_planes
 
 TILE = 64  # target boxes per M2L tile by default (the HIP kernel's widest tile)
 TILE_WIDTHS = (64, 32)  # the tile widths the contraction kernels are built for
+MAX_PLANE_COEFFS = 256  # coefficients of a complex octant translation
 GROUP = 16  # target boxes per octant-translation group (matches the HIP kernel)
 MIN_SLOTS_PER_SPLIT = 12
 
@@ -115,7 +116,12 @@ class _OctantTranslation(E2EBase):
         if not tgt.is_complex():
             return self._apply(actx, kwargs, src, tgt, k)
         # complex (Helmholtz) expansions: the translation is real-linear with
-        # real matrices, applied to the real and the imaginary plane
+        # real matrices; the octant matrices take both planes as they lie, the
+        # per-box kernels one contiguous plane at a time
+        if max(src.shape[1], tgt.shape[1]) <= MAX_PLANE_COEFFS and src.is_contiguous() and \
+                tgt.is_contiguous() and \
+                self._apply(actx, kwargs, src, tgt, k, planes=2) is not None:
+            return tgt
         sr, si = planes(src)
         tr, ti = planes(tgt)
         self._apply(actx, kwargs, sr, tr, k)
@@ -143,15 +149,15 @@ class _OctantTranslation(E2EBase):
         T = out.view(8, n_in, n_out).transpose(1, 2)
         return T*torch.from_numpy(present.astype(np.float64)).to(actx.device)[:, None, None]
 
-    def _launch_octant(self, actx, plan, frag, src, sbase, tgt, tbase):
+    def _launch_octant(self, actx, plan, frag, src, sbase, tgt, tbase, planes=1):
         st, tt = self._tables(actx)
-        flops = 2.0*st.table.nstored*tt.table.nstored*plan["npairs"]
+        flops = 2.0*st.table.nstored*tt.table.nstored*plan["npairs"]*planes
         partial = None
         if self.octant_inputs_per_target > 1:
-            partial = torch.empty(plan["ngroups"]*8*GROUP*tt.table.nstored,
+            partial = torch.empty(plan["ngroups"]*8*GROUP*tt.table.nstored*planes,
                                   dtype=torch.float64, device=tgt.device)
         with kernel_span(self.span_name, flops):
-            _capi.call("sumpyhip_octant_translate", plan["ngroups"],
+            _capi.call("sumpyhip_octant_translate_planes", planes, plan["ngroups"],
                        _capi.ptr(plan["targets"]), _capi.ptr(plan["inputs"]),
                        _capi.ptr(plan["mask"]), int(plan["items"].shape[0]),
                        _capi.ptr(plan["items"]), tt.table.nstored, st.table.nstored,
@@ -254,7 +260,7 @@ class E2EFromChildren(_OctantTranslation):
         plans[key] = plan
         return plan
 
-    def _apply(self, actx, kwargs, src, tgt, k):
+    def _apply(self, actx, kwargs, src, tgt, k, planes=1):
         st, tt = self._tables(actx, kwargs["src_rscale"], kwargs["tgt_rscale"], k)
         centers = kwargs["centers"].contiguous()
         tb = as_i32(kwargs["target_boxes"])
@@ -274,7 +280,9 @@ class E2EFromChildren(_OctantTranslation):
                 return self._launch_octant(actx, dict(plan["dev"], ngroups=plan["ngroups"],
                                                       npairs=plan["npairs"]),
                                            frag, src, kwargs["src_base_ibox"], tgt,
-                                           kwargs["tgt_base_ibox"])
+                                           kwargs["tgt_base_ibox"], planes)
+        if planes > 1:
+            return None
         with kernel_span(self.span_name, 0.0):
             _capi.call("sumpyhip_m2m", kernel_id(self.tgt_expansion.kernel), st.desc,
                        tt.desc, int(tb.shape[0]), _capi.ptr(tb), _capi.ptr(child),
@@ -341,7 +349,7 @@ class E2EFromParent(_OctantTranslation):
         plans[key] = plan
         return plan
 
-    def _apply(self, actx, kwargs, src, tgt, k):
+    def _apply(self, actx, kwargs, src, tgt, k, planes=1):
         st, tt = self._tables(actx, kwargs["src_rscale"], kwargs["tgt_rscale"], k)
         centers = kwargs["centers"].contiguous()
         tb = as_i32(kwargs["target_boxes"])
@@ -361,7 +369,9 @@ class E2EFromParent(_OctantTranslation):
                 return self._launch_octant(actx, dict(plan["dev"], ngroups=plan["ngroups"],
                                                       npairs=plan["npairs"]),
                                            frag, src, kwargs["src_base_ibox"], tgt,
-                                           kwargs["tgt_base_ibox"])
+                                           kwargs["tgt_base_ibox"], planes)
+        if planes > 1:
+            return None
         with kernel_span(self.span_name, 0.0):
             _capi.call("sumpyhip_l2l", kernel_id(self.tgt_expansion.kernel), st.desc,
                        tt.desc, int(tb.shape[0]), _capi.ptr(tb), _capi.ptr(parents),
