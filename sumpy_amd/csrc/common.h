@@ -37,6 +37,14 @@ __device__ __forceinline__ double group_sum(double v, int g) {
   return v;
 }
 
+// orders a wave's LDS accesses: the wave's writes before are seen by its lanes'
+// reads after (no block barrier)
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace sumpyhip
 
 #define SUMPY_REQUIRE(cond, ...)                                   \

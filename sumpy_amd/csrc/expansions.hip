@@ -38,13 +38,6 @@ __device__ __forceinline__ double inv_fact(int n) {
   return 1.0/f;
 }
 
-// LDS written by some lanes of a wave and read by others of the same wave
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // {{{ P2M
 
 // rscale per tree level, for launches that span several levels (a box's

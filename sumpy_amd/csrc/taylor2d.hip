@@ -589,6 +589,115 @@ __global__ __launch_bounds__(TTH) void t2_m2l(T2E es, T2E et, cplx k, const int 
             cscale(acc, ipow(tgt_rscale/src_rscale, tx + ty)));
 }
 
+// The same with class data and at most 64 coefficients: one target box per
+// block, whose groups of G lanes (a lane per target coefficient) take every
+// NG-th source of the list; their sums are added in group order.  A group keeps
+// the class's derivatives in LDS on a grid, entry mx S + my, where t + s is a
+// sum of offsets.  Bound: the latency of a source's loads (27 sources a target
+// on a uniform tree); with a source at a time per block, the five levels of
+// 131072 points at order 10 took 303 us, this way 97 us.
+template <int KIND>
+struct Val {  // a coefficient: real or complex
+  typedef double type;
+  static __device__ __forceinline__ double ld(const double *p, int i) { return p[i]; }
+  static __device__ __forceinline__ double mad(double a, double b, double c) { return c + a*b; }
+  static __device__ __forceinline__ cplx full(double a) { return {a, 0.0}; }
+  static __device__ __forceinline__ double add(double a, double b) { return a + b; }
+  static __device__ __forceinline__ double zero() { return 0.0; }
+};
+template <>
+struct Val<1> {
+  typedef cplx type;
+  static __device__ __forceinline__ cplx ld(const double *p, int i) {
+    return {p[2*i], p[2*i + 1]};
+  }
+  static __device__ __forceinline__ cplx mad(cplx a, cplx b, cplx c) { return cfma(a, b, c); }
+  static __device__ __forceinline__ cplx full(cplx a) { return a; }
+  static __device__ __forceinline__ cplx add(cplx a, cplx b) { return cadd(a, b); }
+  static __device__ __forceinline__ cplx zero() { return {0.0, 0.0}; }
+};
+
+constexpr int MTH = 256;                       // threads per block
+constexpr int TGRID = (2*TPMAX + 1)*(2*TPMAX + 1);
+
+template <int KIND, int G>
+__global__ __launch_bounds__(MTH) void t2_m2l_classes(
+    T2E es, T2E et, const int *target_boxes, const int *starts, const int *lists,
+    const int *classes, int class_start, const double *data, double src_rscale,
+    double tgt_rscale, const double *src, int sbase, double *tgt, int tbase) {
+  typedef Val<KIND> V;
+  typedef typename V::type val;
+  constexpr int NG = MTH/G, CM = KIND == 1 ? 2 : 1;
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int N = es.order + et.order, nd = nfull(N), S = N + 1;
+  // (compressed sets have m_x <= 1 each)
+  const int ngrid = es.compressed && et.compressed ? min(3, S)*S : S*S;
+  val *Dg = reinterpret_cast<val *>(lds);                          // [NG][ngrid]
+  val *Mg = Dg + NG*ngrid;                                         // [NG][G]
+  int *grid_of = reinterpret_cast<int *>(Mg + NG*G);               // [nd]
+  int *off_s = grid_of + nd;                                       // [G]
+  const int it = blockIdx.x, box = target_boxes[it];
+  const int lane = threadIdx.x % G, g = threadIdx.x/G;
+  for (int e = threadIdx.x; e < nd; e += MTH) {
+    int mx, my;
+    untri(e, mx, my);
+    const int at = mx*S + my;
+    grid_of[e] = at < ngrid ? at : -1;
+  }
+  if (threadIdx.x < es.nstored)
+    off_s[threadIdx.x] = es.smx[threadIdx.x]*S + es.smy[threadIdx.x];
+  __syncthreads();
+  const bool act = lane < et.nstored;
+  const int tx = act ? et.smx[lane] : 0, ty = act ? et.smy[lane] : 0;
+  val *D = Dg + g*ngrid, *M = Mg + g*G;
+  const val *Dt = D + tx*S + ty;
+  val acc = V::zero();
+  for (int q = starts[it] + g; q < starts[it + 1]; q += NG) {
+    const double *row = src + (size_t)(lists[q] - sbase)*es.nstored*CM;
+    const double *crow = data + (size_t)(classes[q] - class_start)*nd*CM;
+    if (lane < es.nstored) M[lane] = V::ld(row, lane);
+    for (int e = lane; e < nd; e += G) {
+      const val d = V::ld(crow, e);
+      const int at = grid_of[e];
+      if (at >= 0) D[at] = d;
+    }
+    wave_sync();
+    if (act)
+      #pragma unroll 4
+      for (int s = 0; s < es.nstored; ++s) acc = V::mad(M[s], Dt[off_s[s]], acc);
+    wave_sync();
+  }
+  __syncthreads();
+  Mg[g*G + lane] = acc;
+  __syncthreads();
+  if (g > 0 || !act) return;
+  for (int h = 1; h < NG; ++h) acc = V::add(acc, Mg[h*G + lane]);
+  stv<KIND == 1>(tgt + (size_t)(box - tbase)*et.nstored*CM, lane,
+                 cscale(V::full(acc), ipow(tgt_rscale/src_rscale, tx + ty)));
+}
+
+template <int KIND, int G>
+int launch_m2l_classes(const T2E &es, const T2E &et, int ntgt, const int *target_boxes,
+                       const int *starts, const int *lists, const int *classes, int class_start,
+                       const double *data, double src_rscale, double tgt_rscale,
+                       const double *src, int sbase, double *tgt, int tbase, hipStream_t st) {
+  const int N = es.order + et.order, S = N + 1;
+  const int ngrid = es.compressed && et.compressed ? (S < 3 ? S : 3)*S : S*S;
+  const size_t lds = (size_t)MTH/G*(ngrid + G)*sizeof(typename Val<KIND>::type) +
+                     sizeof(int)*((N + 1)*(N + 2)/2 + G);
+  if (lds > 64*1024) {
+    hipError_t e = hipFuncSetAttribute((const void *)t2_m2l_classes<KIND, G>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess)
+      return set_error(SUMPYHIP_EHIP, "t2d_m2l: cannot raise LDS limit to %zu: %s", lds,
+                       hipGetErrorString(e));
+  }
+  t2_m2l_classes<KIND, G><<<ntgt, MTH, lds, st>>>(es, et, target_boxes, starts, lists, classes,
+                                                  class_start, data, src_rscale, tgt_rscale, src,
+                                                  sbase, tgt, tbase);
+  return check_launch("t2d_m2l");
+}
+
 // }}}
 
 int check_expn(const sumpyhip_t2d_expn *e, const char *what) {
@@ -844,6 +953,17 @@ extern "C" int sumpyhip_t2d_m2l(int kind, const sumpyhip_t2d_expn *src_ex,
                 "t2d_m2l: bad arguments");
   SUMPY_REQUIRE(!class_data || classes, "t2d_m2l: class data without class lists");
   hipStream_t st = (hipStream_t)stream;
+  const int widest = src_ex->nstored > tgt_ex->nstored ? src_ex->nstored : tgt_ex->nstored;
+  if (class_data && widest <= 64) {
+#define M2L_CLASSES(KIND, G)                                                            \
+  launch_m2l_classes<KIND, G>(to_t2e(src_ex), to_t2e(tgt_ex), ntgt, target_boxes,       \
+                              src_box_starts, src_box_lists, classes, class_start,      \
+                              class_data, src_rscale, tgt_rscale, src_expansions,       \
+                              src_base_ibox, tgt_expansions, tgt_base_ibox, st)
+    if (widest <= 32) return kind ? M2L_CLASSES(1, 32) : M2L_CLASSES(0, 32);
+    return kind ? M2L_CLASSES(1, 64) : M2L_CLASSES(0, 64);
+#undef M2L_CLASSES
+  }
   if (kind)
     t2_m2l<1><<<ntgt, TTH, 0, st>>>(to_t2e(src_ex), to_t2e(tgt_ex), kk, target_boxes,
                                     src_box_starts, src_box_lists, classes, class_start,
