@@ -200,12 +200,14 @@ def _octant_items(mask):
     return (g*8 + o).astype(np.int32)
 
 
-def _groups(actx, targets, inputs, labels):
-    """Groups of GROUP targets sharing one label each (inputs[i] feeds target
-    i through octant labels[i]); M2M passes all eight octants per target."""
-    def dev(a):
-        return torch.from_numpy(np.ascontiguousarray(a, np.int32)).to(actx.device)
-    return dev(targets), dev(inputs)
+def _plan_arrays(actx, plan):
+    """The plan's arrays on the device (one upload): groups of GROUP targets
+    sharing one label each (inputs[i] feeds target i through octant
+    labels[i]; M2M passes all eight octants per target)."""
+    arrays = {name: np.ravel(plan[name]) for name in ("targets", "inputs", "mask")}
+    arrays["items"] = _octant_items(plan["mask"])
+    flat = torch.from_numpy(np.concatenate(list(arrays.values())).astype(np.int32))
+    return dict(zip(arrays, flat.to(actx.device).split([len(a) for a in arrays.values()])))
 
 
 class E2EFromChildren(_OctantTranslation):
@@ -271,10 +273,7 @@ class E2EFromChildren(_OctantTranslation):
             if plan is not None:
                 self.last_call_used_octant_matrices = True
                 if "dev" not in plan:
-                    plan["dev"] = dict(zip(("targets", "inputs"), _groups(
-                        actx, plan["targets"], plan["inputs"], None)),
-                        mask=actx.from_numpy(plan["mask"].astype(np.int32)),
-                        items=actx.from_numpy(_octant_items(plan["mask"])))
+                    plan["dev"] = _plan_arrays(actx, plan)
                 frag = self._matrices(actx, plan["offsets"], plan["present"],
                                       kwargs["src_rscale"], kwargs["tgt_rscale"], k)
                 return self._launch_octant(actx, dict(plan["dev"], ngroups=plan["ngroups"],
@@ -328,23 +327,20 @@ class E2EFromParent(_OctantTranslation):
         common = _common_offsets(d, labels) if len(tb) and (pb != tb).all() else None
         plan = None
         if common is not None:
+            # octant by octant in box order, GROUP targets to a group
             order = np.argsort(labels, kind="stable")
             cnt = np.bincount(labels, minlength=8)
-            first = np.concatenate([[0], np.cumsum(cnt)[:-1]])
-            tg, ip, mk = [], [], []
-            for o in range(8):
-                sel = order[first[o]:first[o] + cnt[o]]
-                for c0 in range(0, len(sel), GROUP):
-                    part = sel[c0:c0 + GROUP]
-                    t = np.full(GROUP, -1, np.int64)
-                    t[:len(part)] = tb[part]
-                    i = np.full((8, GROUP), -1, np.int64)
-                    i[o, :len(part)] = pb[part]
-                    tg.append(t)
-                    ip.append(i)
-                    mk.append(1 << o)
-            plan = dict(ngroups=len(tg), targets=np.concatenate(tg),
-                        inputs=np.stack(ip), mask=np.array(mk), offsets=common[0],
+            ngr = -(-cnt//GROUP)
+            lab = labels[order]
+            rank = np.arange(len(tb)) - (np.cumsum(cnt) - cnt)[lab]
+            grp, col = (np.cumsum(ngr) - ngr)[lab] + rank//GROUP, rank % GROUP
+            ng = int(ngr.sum())
+            targets = np.full((ng, GROUP), -1, np.int64)
+            targets[grp, col] = tb[order]
+            inputs = np.full((ng, 8, GROUP), -1, np.int64)
+            inputs[grp, lab, col] = pb[order]
+            plan = dict(ngroups=ng, targets=targets.ravel(), inputs=inputs,
+                        mask=np.repeat(1 << np.arange(8), ngr), offsets=common[0],
                         present=common[1], npairs=len(tb))
         plans[key] = plan
         return plan
@@ -360,10 +356,7 @@ class E2EFromParent(_OctantTranslation):
             if plan is not None:
                 self.last_call_used_octant_matrices = True
                 if "dev" not in plan:
-                    plan["dev"] = dict(zip(("targets", "inputs"), _groups(
-                        actx, plan["targets"], plan["inputs"], None)),
-                        mask=actx.from_numpy(plan["mask"].astype(np.int32)),
-                        items=actx.from_numpy(_octant_items(plan["mask"])))
+                    plan["dev"] = _plan_arrays(actx, plan)
                 frag = self._matrices(actx, plan["offsets"], plan["present"],
                                       kwargs["src_rscale"], kwargs["tgt_rscale"], k)
                 return self._launch_octant(actx, dict(plan["dev"], ngroups=plan["ngroups"],

@@ -265,21 +265,12 @@ def build_device(actx, sources, targets=None, max_particles_in_box=30, max_level
                    _capi.ptr(used), st)
     used_h = used.view(nlevels, nslots).cpu().numpy() > 0
     slot_to_cls = np.full((nlevels, nslots), -1, np.int32)
-    gid = 0
-    cls_ls = np.zeros(nlevels + 1, np.int32)
-    vecs = []
-    for lev in range(nlevels):
-        cls_ls[lev] = gid
-        h = ext/float(1 << lev)
-        for s_ in np.nonzero(used_h[lev])[0]:
-            slot_to_cls[lev, s_] = gid
-            gid += 1
-            rem, v = int(s_), [0]*dim
-            for d in range(dim - 1, -1, -1):
-                v[d] = rem % 7 - 3
-                rem //= 7
-            vecs.append([v[d]*h for d in range(dim)])
-    cls_ls[nlevels] = gid
+    # classes numbered level by level in slot order; slot digits -3..3 base 7
+    lev_of, slot_of = np.nonzero(used_h)
+    slot_to_cls[lev_of, slot_of] = np.arange(len(lev_of))
+    cls_ls = np.searchsorted(lev_of, np.arange(nlevels + 1)).astype(np.int32)
+    digits = np.stack([slot_of//7**(dim - 1 - d) % 7 - 3 for d in range(dim)], axis=1)
+    vecs = digits*(ext/(1 << lev_of).astype(np.float64))[:, None]
     entry_level = _i32(torch.repeat_interleave(box_levels[totp], c2.to(torch.int64)))
     cls = torch.empty(n2, dtype=_I32, device=dev)
     s2c = torch.from_numpy(slot_to_cls.ravel()).to(dev)
@@ -289,7 +280,7 @@ def build_device(actx, sources, targets=None, max_particles_in_box=30, max_level
     vh["from_sep_siblings_translation_classes"] = cls
     vh["from_sep_siblings_translation_classes_level_starts"] = torch.from_numpy(cls_ls).to(dev)
     vh["from_sep_siblings_translation_class_to_distance_vector"] = torch.tensor(
-        np.array(vecs, np.float64).reshape(-1, dim).T.copy(), device=dev)
+        vecs.reshape(-1, dim).T.copy(), device=dev)
     # list 3, per source level
     nt = int(tb.numel())
     c3 = two_pass(3, tb, nlevels).view(nt, nlevels)
@@ -298,13 +289,16 @@ def build_device(actx, sources, targets=None, max_particles_in_box=30, max_level
     if l3.numel():
         _capi.call("sumpytree_gpu_list", 3, *view, _capi.ptr(coll), nt, _capi.ptr(tb), None,
                    _capi.ptr(off), _capi.ptr(l3), None, None, st)
-    sep = []
-    off_h = off.cpu().numpy()
-    for lev in range(nlevels):
-        cl = c3[:, lev]
-        sel = torch.nonzero(cl).flatten()
-        a, b = int(off_h[lev*nt]), int(off_h[(lev + 1)*nt])
-        sep.append((_i32(tb[sel]), _excl(cl[sel]), l3[a:b]))
+    # target boxes with a list 3 by source level: all levels in one selection
+    c3t = c3.t().contiguous()
+    sel = torch.nonzero(c3t.view(-1)).flatten()
+    cuts = torch.searchsorted(sel, torch.arange(nlevels + 1, device=dev)*nt)
+    cuts, ends = torch.stack([cuts, off[::max(nt, 1)][:nlevels + 1].long()]).tolist() if nt \
+        else ([0]*(nlevels + 1),)*2
+    boxes3 = tb[sel % max(nt, 1)] if nt else tb[:0]
+    upto = _excl(c3t.view(-1)[sel])
+    sep = [(boxes3[i:j], upto[i:j + 1] - upto[i], l3[a:b])
+           for i, j, a, b in zip(cuts, cuts[1:], ends, ends[1:])]
     vh["sep_smaller"] = sep
     # list 4
     c4 = two_pass(4, totp)
