@@ -268,13 +268,9 @@ __global__ __launch_bounds__(64) void m2p_helm3d(
 //   sum_s M_s d^s H = sum_a x^a sum_n g_{a+n} R_{a,n}(y, z),
 //   R_{a,n} = sum_{beta + gamma <= n} C[a,n,beta,gamma] y^beta z^gamma,
 //   C[a,n,beta,gamma] = sum_{j=beta}^{n-gamma} M_(a, 2j-beta, 2(n-j)-gamma)
-//                       h(2j-beta, j) h(2(n-j)-gamma, n-j)   (|m| <= p only).
-// The coefficients depend on the multipole only: the wave forms them once per
-// source box in LDS, then every lane evaluates the polynomials at its target
-// by Horner's rule with compile-time offsets (broadcast LDS reads).
-// Coefficient order: a, then n, then beta, then gamma.
-
-__host__ __device__ constexpr int tet(int n) { return n*(n + 1)*(n + 2)/6; }
+//                       h(2j-beta, j) h(2(n-j)-gamma, n-j).
+// All M of the sum have the degree a + 2n - beta - gamma, so C vanishes unless
+// gamma >= 2n + a - p - beta: 455 of the 819 remain at order 12.
 
 // 2-vector of T (the complex terms of the FP32 list-3/4 forms)
 template <typename T>
@@ -284,137 +280,271 @@ struct V2T<float> { typedef float2 type; };
 template <typename T>
 __device__ __forceinline__ typename V2T<T>::type mk2(T a, T b) { return {a, b}; }
 
+// The layout of C (and of the moments of P2L): a, then n, then beta, then
+// gamma from the first one that does not vanish for a = 0.  Both halves have
+// that shape, the entries that vanish for a = 1 only stay zero.
 template <int ORD>
-struct M2PPoly {
-  static constexpr int N0 = tet(ORD + 1);   // coefficients with a = 0
-  static constexpr int NC = N0 + tet(ORD);  // all
+struct HelmPoly {
+  // first gamma of the row (a, n, beta)
+  __host__ __device__ static constexpr int lo(int a, int n, int b) {
+    const int v = 2*n + a - ORD - b;
+    return v > 0 ? v : 0;
+  }
+  // row (n, beta) within n's rows; beta = n + 1: their size
+  __host__ __device__ static constexpr int row(int n, int b) {
+    const int k = 2*n > ORD ? 2*n - ORD : 0;
+    return b*(n + 1 - k) - (b > k ? (b - k)*(b - k - 1)/2 : 0);
+  }
+  __host__ __device__ static constexpr int base(int n) {
+    int v = 0;
+    for (int i = 0; i < n; ++i) v += row(i, i + 1);
+    return v;
+  }
+  static constexpr int NA = base(ORD + 1);  // one half
+  static constexpr int NC = 2*NA;
+  static constexpr int RL = ORD/2 + 1;      // longest row
+  static constexpr int NR = (NC + 63)/64;   // coefficients of a lane
+  static constexpr int NS = (ORD + 1)*(ORD + 1);
 };
 
 // stored index of (a, b, c) in the PDE-compressed order (degree d = a+b+c:
 // first a = 0 with b = 0..d, then a = 1 with b = 0..d-1)
-__device__ __forceinline__ int stored_index(int a, int b, int c) {
+__host__ __device__ constexpr int stored_index(int a, int b, int c) {
   const int d = a + b + c;
   return d*d + (a ? d + 1 + b : b);
 }
 
-template <int ORD, typename T>
-__device__ __forceinline__ void m2p_poly_eval(const typename V2T<T>::type *C, T x, T y, T z,
-                                              const T *gr, const T *gi, T &pr, T &pi) {
-  #pragma unroll
-  for (int a = 0; a <= 1; ++a) {
-    const int base = a ? M2PPoly<ORD>::N0 : 0;
-    T ar = 0, ai = 0;
-    #pragma unroll
-    for (int n = 0; n <= ORD - a; ++n) {
-      T Rr = 0, Ri = 0;
-      #pragma unroll
-      for (int b = n; b >= 0; --b) {
-        T Sr = 0, Si = 0;
-        #pragma unroll
-        for (int c = n - b; c >= 0; --c) {
-          const auto v = C[base + tet(n) + b*(n + 1) - b*(b - 1)/2 + c];
-          Sr = Sr*z + v.x;
-          Si = Si*z + v.y;
+// h(n, i), ceil(n/2) <= i <= n (exact in double for n <= 12)
+constexpr double herm(int n, int i) {
+  double h = 1;
+  for (int o = 3; o <= n; o += 2) h *= o;
+  for (int q = (n + 1)/2; q < i; ++q) h = h*(2*(n - q))/double((2*q + 2 - n)*(2*q + 1 - n));
+  return h;
+}
+
+// Per coefficient the stored terms that it sums.  Coefficients are dealt to
+// the lanes by falling number of terms (round r, lane l: the r 64 + l-th), so
+// that a wave's lanes end together.
+template <int ORD>
+struct HelmRounds {
+  int terms[HelmPoly<ORD>::NR];  // of the round's longest
+  int first[HelmPoly<ORD>::NR];  // slot of its first term
+  int slots;
+};
+template <int ORD>
+constexpr int helm_nterms(int a, int n, int b, int c) {
+  return c >= HelmPoly<ORD>::lo(a, n, b) && a + n <= ORD ? n - b - c + 1 : 0;
+}
+template <int ORD>
+constexpr HelmRounds<ORD> helm_rounds() {
+  HelmRounds<ORD> r{};
+  int count[ORD + 2] = {};
+  for (int a = 0; a < 2; ++a)
+    for (int n = 0; n <= ORD; ++n)
+      for (int b = 0; b <= n; ++b)
+        for (int c = HelmPoly<ORD>::lo(0, n, b); c <= n - b; ++c)
+          ++count[helm_nterms<ORD>(a, n, b, c)];
+  int at = 0;
+  for (int t = ORD + 1; t >= 0; --t)
+    for (int k = 0; k < count[t]; ++k, ++at)
+      if (at % 64 == 0) r.terms[at/64] = t;
+  for (int k = 0; k < HelmPoly<ORD>::NR; ++k) {
+    r.first[k] = r.slots;
+    r.slots += r.terms[k];
+  }
+  return r;
+}
+template <int ORD>
+constexpr HelmRounds<ORD> HELM_ROUNDS = helm_rounds<ORD>();
+
+template <int ORD>
+struct HelmTerms {
+  double w[HELM_ROUNDS<ORD>.slots][64];
+  unsigned char src[HELM_ROUNDS<ORD>.slots][64];  // stored index; no term: NS, a zero
+  unsigned short pos[HelmPoly<ORD>::NR][64];      // in C; no coefficient: NC, not read
+};
+template <int ORD>
+constexpr HelmTerms<ORD> helm_terms() {
+  typedef HelmPoly<ORD> P;
+  HelmTerms<ORD> t{};
+  for (int l = 0; l < 64; ++l) {
+    for (int r = 0; r < P::NR; ++r) t.pos[r][l] = P::NC;
+    for (int s = 0; s < HELM_ROUNDS<ORD>.slots; ++s) t.src[s][l] = P::NS;
+  }
+  int count[ORD + 2] = {}, next[ORD + 2] = {};
+  for (int a = 0; a < 2; ++a)
+    for (int n = 0; n <= ORD; ++n)
+      for (int b = 0; b <= n; ++b)
+        for (int c = P::lo(0, n, b); c <= n - b; ++c) ++count[helm_nterms<ORD>(a, n, b, c)];
+  for (int k = ORD, at = 0; k >= 0; --k) next[k] = at += count[k + 1];
+  for (int a = 0; a < 2; ++a)
+    for (int n = 0, o = 0; n <= ORD; ++n)
+      for (int b = 0; b <= n; ++b)
+        for (int c = P::lo(0, n, b); c <= n - b; ++c, ++o) {
+          const int nt = helm_nterms<ORD>(a, n, b, c), at = next[nt]++;
+          const int r = at/64, l = at % 64;
+          t.pos[r][l] = (unsigned short)(a*P::NA + o);
+          for (int m = 0; m < nt; ++m) {
+            const int j = b + m, bb = 2*j - b, cc = 2*(n - j) - c, s = HELM_ROUNDS<ORD>.first[r] + m;
+            t.w[s][l] = herm(bb, j)*herm(cc, n - j);
+            t.src[s][l] = (unsigned char)stored_index(a, bb, cc);
+          }
         }
-        Rr = Rr*y + Sr;
-        Ri = Ri*y + Si;
+  return t;
+}
+template <int ORD>
+__device__ const HelmTerms<ORD> HELM_TERMS = helm_terms<ORD>();
+
+// sum_n g_{a+n} R_{a,n}(y, z) from C's half of a; zp[e] = z^e; g gives g_{a+n}
+template <int ORD, typename T, typename G>
+__device__ __forceinline__ void m2p_poly_eval(const typename V2T<T>::type *C, T y, T z,
+                                              const T *zp, G &&g, T &ar, T &ai) {
+  typedef HelmPoly<ORD> P;
+  #pragma unroll
+  for (int n = 0; n <= ORD; ++n) {
+    T Rr = 0, Ri = 0;
+    #pragma unroll
+    for (int b = n; b >= 0; --b) {
+      const int lo = P::lo(0, n, b), off = P::base(n) + P::row(n, b) - lo;
+      T Sr = C[off + n - b].x, Si = C[off + n - b].y;
+      #pragma unroll
+      for (int c = n - b - 1; c >= lo; --c) {
+        const auto v = C[off + c];
+        Sr = Sr*z + v.x;
+        Si = Si*z + v.y;
       }
-      ar += gr[a + n]*Rr - gi[a + n]*Ri;
-      ai += gr[a + n]*Ri + gi[a + n]*Rr;
+      if (lo) { Sr *= zp[lo]; Si *= zp[lo]; }
+      Rr = b == n ? Sr : Rr*y + Sr;
+      Ri = b == n ? Si : Ri*y + Si;
     }
-    if (a == 0) { pr += ar; pi += ai; } else { pr += x*ar; pi += x*ai; }
+    T gr, gi;
+    g(n, gr, gi);
+    ar += gr*Rr - gi*Ri;
+    ai += gr*Ri + gi*Rr;
+    __builtin_amdgcn_sched_barrier(0);  // no reads of C far ahead: registers
   }
 }
 
+// One block of NW waves per target box, lane = target, each wave on every
+// NW-th source box: it forms C from the box's multipole in LDS and evaluates
+// the polynomials by Horner's rule with compile-time offsets (broadcast LDS
+// reads).  Where a box has at most 32 targets, the two halves of the wave take
+// a = 0 and a = 1 of the same targets.  The waves' sums are added in order.
+// The pairs of one box are independent: one wave took them in turn, 21 us
+// each, 45 in a row (150000 points on a sphere, order 12, FP32: 2.45 ms in
+// three launches, this way 0.37 ms).  Bound by the LDS reads of C and the FP64
+// g_q of every target.
 // T = float: the polynomial, its coefficients and g_q in FP32 (g_q from FP64
 // values), each source box's term added to FP64 sums
+template <typename T>
+constexpr int M2PH_NW = sizeof(T) == 4 ? 8 : 4;
+
 template <int ORD, typename T>
-__global__ __launch_bounds__(64) void m2p_helm3d_poly(
-    double k, int ntgt, const int *target_boxes, const int *starts, const int *lists,
-    const int *bts, const int *btc, const double *centers, int nboxes, const double *tx,
-    const double *ty, const double *tz, double rscale, double scale, const double2 *src,
-    int sbase, double2 *pot) {
-  constexpr int NC = M2PPoly<ORD>::NC, NS = (ORD + 1)*(ORD + 1), HS = ORD + 1;
-  __shared__ typename V2T<T>::type sC[NC];
-  __shared__ double2 sM[NS];
-  __shared__ double ht[HS*HS];
-  __shared__ unsigned dec[NC];
-  herm_table(ht, ORD);
-  const int lane = threadIdx.x;
-  for (int i = lane; i < NC; i += 64) {  // (a, n, beta, gamma) of coefficient i
-    const int a = i >= M2PPoly<ORD>::N0, r = a ? i - M2PPoly<ORD>::N0 : i;
-    int n = 0;
-    while (tet(n + 1) <= r) ++n;
-    int q = r - tet(n), b = 0;
-    while (q >= n + 1 - b) { q -= n + 1 - b; ++b; }
-    dec[i] = a | (n << 1) | (b << 8) | (q << 16);
-  }
+__global__ __launch_bounds__(64*M2PH_NW<T>, sizeof(T) == 4 ? 4 : 2) void m2p_helm3d_poly(
+    double k, int ntgt, const int *__restrict__ target_boxes, const int *__restrict__ starts,
+    const int *__restrict__ lists, const int *__restrict__ bts, const int *__restrict__ btc,
+    const double *__restrict__ centers, int nboxes, const double *__restrict__ tx,
+    const double *__restrict__ ty, const double *__restrict__ tz, double rscale, double scale,
+    const double2 *__restrict__ src, int sbase, double2 *pot) {
+  typedef HelmPoly<ORD> P;
+  constexpr int NS = P::NS, NW = M2PH_NW<T>, NM = (NS + 63)/64;
+  __shared__ typename V2T<T>::type sC[NW][P::NC + 2];
+  __shared__ double2 sM[NW][NS > 63 ? NS + 1 : 64];  // at the end: the waves' sums
+  const HelmTerms<ORD> &terms = HELM_TERMS<ORD>;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const double rinv = 1.0/rscale, kappa = k*rscale;
   for (int ib = blockIdx.x; ib < ntgt; ib += gridDim.x) {
+    const int i0 = starts[ib], i1 = starts[ib + 1];
     const int tb = target_boxes[ib];
     const int t0 = bts[tb], nt = btc[tb];
     for (int tc = 0; tc < nt; tc += 64) {
-      const bool valid = tc + lane < nt;
-      const int t = t0 + tc + (valid ? lane : 0);
+      const bool split = nt - tc <= 32;
+      const int half = split ? lane >> 5 : 0, tl = split ? lane & 31 : lane;
+      const int t = t0 + tc + (tc + tl < nt ? tl : 0);
       const double X = tx[t], Y = ty[t], Z = tz[t];
       double pr = 0, pi = 0;
-      for (int qq = starts[ib]; qq < starts[ib + 1]; ++qq) {
-        const int sb = lists[qq];
-        __syncthreads();  // previous source box done with sC / sM
-        const double2 *M = src + (size_t)(sb - sbase)*NS;
-        for (int u = lane; u < NS; u += 64) sM[u] = M[u];
-        __syncthreads();
-        for (int i = lane; i < NC; i += 64) {
-          const unsigned d = dec[i];
-          const int a = d & 1, n = (d >> 1) & 127, be = (d >> 8) & 255, ga = d >> 16;
+      double2 m[NM];
+      auto load = [&](int q) {
+        const double2 *M = src + (size_t)(lists[q] - sbase)*NS;
+        #pragma unroll
+        for (int u = 0; u < NM; ++u) m[u] = M[min(lane + 64*u, NS - 1)];
+      };
+      if (i0 + wave < i1) load(i0 + wave);
+      for (int q = i0 + wave; q < i1; q += NW) {
+        const int sb = lists[q];
+        wave_sync();  // the previous box's C and M are read
+        #pragma unroll
+        for (int u = 0; u < NM; ++u)
+          if (lane + 64*u < NS) sM[wave][lane + 64*u] = m[u];
+        if (lane == 0) sM[wave][NS] = make_double2(0, 0);
+        wave_sync();
+        if (q + NW < i1) load(q + NW);
+        #pragma unroll
+        for (int r = 0; r < P::NR; ++r) {
           double vr = 0, vi = 0;
-          for (int j = be; j <= n - ga; ++j) {
-            const int b = 2*j - be, c = 2*(n - j) - ga;
-            if (a + b + c > ORD) continue;
-            const double w = ht[b*HS + j]*ht[c*HS + (n - j)];
-            const double2 m = sM[stored_index(a, b, c)];
-            vr += w*m.x;
-            vi += w*m.y;
+          #pragma unroll
+          for (int s = HELM_ROUNDS<ORD>.first[r];
+               s < HELM_ROUNDS<ORD>.first[r] + HELM_ROUNDS<ORD>.terms[r]; ++s) {
+            const double w = terms.w[s][lane];
+            const double2 v = sM[wave][terms.src[s][lane]];
+            vr += w*v.x;
+            vi += w*v.y;
           }
-          sC[i] = mk2<T>(T(vr), T(vi));
+          sC[wave][terms.pos[r][lane]] = mk2<T>(T(vr), T(vi));
         }
         const double x = (X - centers[sb])*rinv, y = (Y - centers[nboxes + sb])*rinv,
                      z = (Z - centers[2*(size_t)nboxes + sb])*rinv;
-        double gr[ORD + 1], gi[ORD + 1];
+        T gr[ORD + 1], gi[ORD + 1], zp[ORD + 1];
         {
           const double r = sqrt(x*x + y*y + z*z), ri = 1.0/r, ri2 = ri*ri;
           double sn, cs;
           sincos(kappa*r, &sn, &cs);
-          gr[0] = cs*ri;
-          gi[0] = sn*ri;
-          if (ORD >= 1) {
-            const double kr = kappa*r;
-            gr[1] = (-cs - sn*kr)*ri2*ri;
-            gi[1] = (cs*kr - sn)*ri2*ri;
-          }
+          const double kr = kappa*r;
+          double ar = cs*ri, ai = sn*ri, br = (-cs - sn*kr)*ri2*ri, bi = (cs*kr - sn)*ri2*ri;
+          gr[0] = T(ar); gi[0] = T(ai);
+          gr[1] = T(br); gi[1] = T(bi);
           #pragma unroll
-          for (int q = 2; q <= ORD; ++q) {
-            gr[q] = (-(2*q - 1)*gr[q - 1] - kappa*kappa*gr[q - 2])*ri2;
-            gi[q] = (-(2*q - 1)*gi[q - 1] - kappa*kappa*gi[q - 2])*ri2;
+          for (int e = 2; e <= ORD; ++e) {
+            const double cr = (-(2*e - 1)*br - kappa*kappa*ar)*ri2,
+                         ci = (-(2*e - 1)*bi - kappa*kappa*ai)*ri2;
+            gr[e] = T(cr); gi[e] = T(ci);
+            ar = br; ai = bi; br = cr; bi = ci;
           }
+          zp[0] = 1;
+          #pragma unroll
+          for (int e = 1; e <= ORD; ++e) zp[e] = zp[e - 1]*T(z);
         }
-        __syncthreads();
-        if constexpr (sizeof(T) == sizeof(double)) {
-          m2p_poly_eval<ORD, double>(sC, x, y, z, gr, gi, pr, pi);
-        } else {
-          T grt[ORD + 1], git[ORD + 1];
-          #pragma unroll
-          for (int q = 0; q <= ORD; ++q) { grt[q] = T(gr[q]); git[q] = T(gi[q]); }
-          T br = 0, bi = 0;
-          m2p_poly_eval<ORD, T>(sC, T(x), T(y), T(z), grt, git, br, bi);
-          pr += double(br);
-          pi += double(bi);
+        wave_sync();
+        for (int pass = 0; pass < (split ? 1 : 2); ++pass) {
+          const int a = half + pass;
+          T ar = 0, ai = 0;
+          m2p_poly_eval<ORD, T>(sC[wave] + a*P::NA, T(y), T(z), zp, [&](int n, T &u, T &v) {
+            const int n1 = n < ORD ? n + 1 : ORD;  // C(1, ORD, ..) is zero
+            u = a ? gr[n1] : gr[n];
+            v = a ? gi[n1] : gi[n];
+          }, ar, ai);
+          const T f = a ? T(x) : T(1);
+          pr += double(f*ar);
+          pi += double(f*ai);
         }
       }
-      if (valid) {
-        pot[t].x += scale*rinv*pr;
-        pot[t].y += scale*rinv*pi;
+      wave_sync();
+      sM[wave][lane] = make_double2(pr, pi);
+      __syncthreads();
+      if (threadIdx.x < (split ? 32 : 64) && tc + (int)threadIdx.x < nt) {
+        double sr = 0, si = 0;
+        for (int w = 0; w < NW; ++w)
+          for (int h = 0; h <= (split ? 1 : 0); ++h) {
+            const double2 v = sM[w][threadIdx.x + 32*h];
+            sr += v.x;
+            si += v.y;
+          }
+        double2 &o = pot[t0 + tc + threadIdx.x];
+        o.x += scale*rinv*sr;
+        o.y += scale*rinv*si;
       }
+      __syncthreads();
     }
   }
 }
@@ -526,62 +656,103 @@ __global__ __launch_bounds__(256) void p2l_helm3d(
 // The transpose of the polynomial M2P: with xi = (c - y)/rho,
 //   L_(a,b,c) = sum_{j,l} h(b,j) h(c,l) Phi_a(j + l, 2j - b, 2l - c),
 //   Phi_a(n, beta, gamma) = sum_y q_y g_{a+n}(|xi_y|) x_y^a y_y^beta z_y^gamma,
-// (beta + gamma <= n <= p - a), then times 1/rho.  Thread r owns the moment row
-// (a, n, beta) -- (p+1)^2 rows, gamma = 0..n-beta -- in registers while the
-// box's list-4 sources stream through LDS; the coefficients are assembled
-// from the moments at the end.
+// then times 1/rho; only the moments of degree a + 2n - beta - gamma <= p are
+// needed, so that a row (a, n, beta) has at most p/2 + 1 of them.  A thread
+// owns one of the (p+1)^2 rows, in registers, the rows sorted by length: a wave
+// runs to the length of its longest.  The box's list-4 sources stream through
+// LDS in chunks that are filled across the source boxes; rows of the staged
+// terms are padded (threads read different g_q and powers of one source).
+// 150000 points on a sphere, order 12, FP32: 0.83 ms with whole rows, a chunk
+// per source box, this way 0.44 ms.  Bound by the staging of a chunk (FP64 g_q
+// of one wave) and the LDS reads of the powers.
 
-// T = float: the staged terms (q g_q, powers) and each chunk's moment sums
-// in FP32, added to FP64 totals per chunk of CH sources
+template <int ORD>
+struct HelmRowTable {
+  unsigned row[HelmPoly<ORD>::NS];  // a | n << 1 | beta << 8 | length << 16
+};
+template <int ORD>
+constexpr HelmRowTable<ORD> helm_rows() {
+  typedef HelmPoly<ORD> P;
+  HelmRowTable<ORD> t{};
+  int at = 0;
+  for (int len = P::RL; len >= 1; --len)
+    for (int a = 0; a < 2; ++a)
+      for (int n = 0; n <= ORD - a; ++n)
+        for (int b = 0; b <= n; ++b)
+          if (n - b + 1 - P::lo(a, n, b) == len)
+            t.row[at++] = unsigned(a | n << 1 | b << 8 | len << 16);
+  return t;
+}
+template <int ORD>
+__device__ const HelmRowTable<ORD> HELM_ROWS = helm_rows<ORD>();
+
+// T = float: the staged terms (q g_q, powers) and the sums of 32 sources in
+// FP32, added to FP64 totals
 template <int ORD, typename T>
-__global__ __launch_bounds__(256) void p2l_helm3d_moments(
-    double k, int ntgt, const int *target_boxes, const int *starts, const int *lists,
-    const int *bss, const int *bsc, const double *centers, int nboxes, const double *sx,
-    const double *sy, const double *sz, const double2 *w0, double rscale, double2 *tgt,
-    int tbase) {
-  constexpr int NS = (ORD + 1)*(ORD + 1), NC = M2PPoly<ORD>::NC, HS = ORD + 1;
-  constexpr int CH = P2LH_CH, NP = ORD + 1;
-  // the source staging (q g_q, powers) and, after the last source, the
-  // moments share one LDS buffer
+__global__ __launch_bounds__(256, 4) void p2l_helm3d_moments(
+    double k, int ntgt, const int *__restrict__ target_boxes, const int *__restrict__ starts,
+    const int *__restrict__ lists, const int *__restrict__ bss, const int *__restrict__ bsc,
+    const double *__restrict__ centers, int nboxes, const double *__restrict__ sx,
+    const double *__restrict__ sy, const double *__restrict__ sz,
+    const double2 *__restrict__ w0, double rscale, double2 *tgt, int tbase) {
+  typedef HelmPoly<ORD> P;
   typedef typename V2T<T>::type V2;
-  constexpr int STAGE = NP*CH*2 + 2*NP*CH + CH;  // doubles
-  constexpr int BUF = STAGE > 2*NC ? STAGE : 2*NC;
-  __shared__ __align__(16) double sbuf[BUF];
-  V2 (*sQG)[CH] = reinterpret_cast<V2 (*)[CH]>(sbuf);
-  T (*sY)[CH] = reinterpret_cast<T (*)[CH]>(sbuf + NP*CH*2);
-  T (*sZ)[CH] = reinterpret_cast<T (*)[CH]>(sbuf + NP*CH*3);
-  T *sX = reinterpret_cast<T *>(sbuf + NP*CH*4);
+  constexpr int NS = P::NS, HS = ORD + 1, CH = P2LH_CH, CS = CH + 1, NP = ORD + 1, RL = P::RL;
+  // the source staging (q g_q, powers of z, y, x: lanes past the end of their
+  // row read powers of y) and, after the last source, the moments
+  constexpr size_t STAGE = NP*CS*sizeof(V2) + (2*NP + 2)*CS*sizeof(T);
+  constexpr size_t BUF = STAGE > P::NC*sizeof(double2) ? STAGE : P::NC*sizeof(double2);
+  static_assert(RL <= NP, "rows read past the powers");
+  __shared__ __align__(16) char sbuf[BUF];
+  V2 (*sQG)[CS] = reinterpret_cast<V2 (*)[CS]>(sbuf);
+  T (*sZ)[CS] = reinterpret_cast<T (*)[CS]>(sbuf + NP*CS*sizeof(V2));
+  T (*sY)[CS] = sZ + NP;
+  T (*sX)[CS] = sY + NP;  // x^0, x^1
   double2 *sPhi = reinterpret_cast<double2 *>(sbuf);
   __shared__ double ht[HS*HS];
+  __shared__ int sBase[NP];                  // HelmPoly::base
+  __shared__ int sBox[64], sPre[65];         // first source, sources before (64 boxes)
   herm_table(ht, ORD);
-  const int tid = threadIdx.x;
-  // moment row of this thread
-  int ra = 0, rn = 0, rb = 0, rlen = 0, rbase = 0;
-  if (tid < NS) {
-    constexpr int R0 = (ORD + 1)*(ORD + 2)/2;
-    ra = tid >= R0;
-    int r = ra ? tid - R0 : tid;
-    while (r > rn) { r -= rn + 1; ++rn; }
-    rb = r;
-    rlen = rn - rb + 1;
-    rbase = (ra ? M2PPoly<ORD>::N0 : 0) + tet(rn) + rb*(rn + 1) - rb*(rb - 1)/2;
-  }
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (tid < NP) sBase[tid] = P::base(tid);
+  const unsigned row = tid < NS ? HELM_ROWS<ORD>.row[tid] : 0;
+  const int ra = row & 1, rn = (row >> 1) & 127, rb = (row >> 8) & 255, rlen = row >> 16;
+  const int rlo = rlen ? P::lo(ra, rn, rb) : 0;
+  const int wlen = __builtin_amdgcn_readfirstlane(rlen);  // the wave's longest
   const double rinv = 1.0/rscale, kappa = k*rscale;
   for (int ib = blockIdx.x; ib < ntgt; ib += gridDim.x) {
     const int tb = target_boxes[ib];
     const double cx = centers[tb], cy = centers[nboxes + tb],
                  cz = centers[2*(size_t)nboxes + tb];
-    double pr[NP], pi[NP];
+    double pr[RL], pi[RL];
     #pragma unroll
-    for (int g = 0; g < NP; ++g) { pr[g] = 0; pi[g] = 0; }
-    for (int q = starts[ib]; q < starts[ib + 1]; ++q) {
-      const int sbox = lists[q];
-      const int s0 = bss[sbox], ns = bsc[sbox];
-      for (int sc = 0; sc < ns; sc += CH) {
-        const int n = min(CH, ns - sc);
-        __syncthreads();
+    for (int g = 0; g < RL; ++g) { pr[g] = 0; pi[g] = 0; }
+    for (int q0 = starts[ib]; q0 < starts[ib + 1]; q0 += 64) {
+      const int nb = min(64, starts[ib + 1] - q0);
+      __syncthreads();
+      if (tid < 64) {
+        const int sb = tid < nb ? lists[q0 + tid] : 0;
+        int sum = tid < nb ? bsc[sb] : 0;
+        sBox[tid] = tid < nb ? bss[sb] : 0;
+        for (int o = 1; o < 64; o <<= 1) {
+          const int v = __shfl_up(sum, o, 64);
+          if (lane >= o) sum += v;
+        }
+        sPre[tid + 1] = sum;
+        if (tid == 0) sPre[0] = 0;
+      }
+      __syncthreads();
+      const int total = sPre[nb];
+      for (int sc = 0; sc < total; sc += CH) {
+        const int n = min(CH, total - sc);
+        if (sc) __syncthreads();
         if (tid < n) {
-          const int si = s0 + sc + tid;
+          // the last box that starts at or before source sc + tid
+          int bx = 0;
+          #pragma unroll
+          for (int o = 32; o > 0; o >>= 1)
+            if (bx + o < nb && sPre[bx + o] <= sc + tid) bx += o;
+          const int si = sBox[bx] + sc + tid - sPre[bx];
           const double x = (cx - sx[si])*rinv, y = (cy - sy[si])*rinv, z = (cz - sz[si])*rinv;
           const double r = sqrt(x*x + y*y + z*z), ri = 1.0/r, ri2 = ri*ri;
           double sn, cs;
@@ -589,13 +760,9 @@ __global__ __launch_bounds__(256) void p2l_helm3d_moments(
           const double2 w = w0[si];
           double ar = cs*ri, ai = sn*ri;
           sQG[0][tid] = mk2<T>(T(w.x*ar - w.y*ai), T(w.x*ai + w.y*ar));
-          double br = 0, bi = 0;
-          if (ORD >= 1) {
-            const double kr = kappa*r;
-            br = (-cs - sn*kr)*ri2*ri;
-            bi = (cs*kr - sn)*ri2*ri;
-            sQG[1][tid] = mk2<T>(T(w.x*br - w.y*bi), T(w.x*bi + w.y*br));
-          }
+          const double kr = kappa*r;
+          double br = (-cs - sn*kr)*ri2*ri, bi = (cs*kr - sn)*ri2*ri;
+          sQG[1][tid] = mk2<T>(T(w.x*br - w.y*bi), T(w.x*bi + w.y*br));
           #pragma unroll
           for (int g = 2; g <= ORD; ++g) {
             const double f = -(2*g - 1);
@@ -611,67 +778,52 @@ __global__ __launch_bounds__(256) void p2l_helm3d_moments(
             py *= y;
             pz *= z;
           }
-          sX[tid] = T(x);
+          sX[0][tid] = T(1);
+          sX[1][tid] = T(x);
         }
         __syncthreads();
-        if constexpr (sizeof(T) == sizeof(double)) {
-          if (tid < NS) {
-            #pragma unroll 2
-            for (int j = 0; j < n; ++j) {
-              const V2 qg = sQG[ra + rn][j];
-              const double m = (ra ? sX[j] : 1.0)*sY[rb][j];
-              const double wr = qg.x*m, wi = qg.y*m;
-              #pragma unroll
-              for (int g = 0; g < NP; ++g) {
-                if (g < rlen) {
-                  const double zg = sZ[g][j];
-                  pr[g] += wr*zg;
-                  pi[g] += wi*zg;
-                }
-              }
-            }
-          }
-        } else if (tid < NS) {
-          T cr[NP], ci[NP];
+        const V2 *qg = sQG[ra + rn];
+        const T *xs = sX[ra], *ys = sY[rb];
+        for (int j0 = 0; j0 < n; j0 += 32) {
+          T cr[RL], ci[RL];
           #pragma unroll
-          for (int g = 0; g < NP; ++g) { cr[g] = 0; ci[g] = 0; }
+          for (int g = 0; g < RL; ++g) { cr[g] = 0; ci[g] = 0; }
           #pragma unroll 2
-          for (int j = 0; j < n; ++j) {
-            const V2 qg = sQG[ra + rn][j];
-            const T m = (ra ? sX[j] : T(1))*sY[rb][j];
-            const T wr = qg.x*m, wi = qg.y*m;
+          for (int j = j0; j < min(j0 + 32, n); ++j) {
+            const V2 v = qg[j];
+            const T m = xs[j]*ys[j];
+            const T wr = v.x*m, wi = v.y*m;
             #pragma unroll
-            for (int g = 0; g < NP; ++g) {
-              if (g < rlen) {
-                const T zg = sZ[g][j];
+            for (int g = 0; g < RL; ++g) {
+              if (g < wlen) {
+                const T zg = sZ[rlo + g][j];
                 cr[g] += wr*zg;
                 ci[g] += wi*zg;
               }
             }
           }
           #pragma unroll
-          for (int g = 0; g < NP; ++g) { pr[g] += double(cr[g]); pi[g] += double(ci[g]); }
+          for (int g = 0; g < RL; ++g) { pr[g] += double(cr[g]); pi[g] += double(ci[g]); }
         }
       }
     }
     __syncthreads();
-    if (tid < NS) {
-      #pragma unroll
-      for (int g = 0; g < NP; ++g)
-        if (g < rlen) sPhi[rbase + g] = make_double2(pr[g], pi[g]);
-    }
+    #pragma unroll
+    for (int g = 0; g < RL; ++g)
+      if (g < rlen)
+        sPhi[ra*P::NA + sBase[rn] + P::row(rn, rb) + rlo - P::lo(0, rn, rb) + g] =
+            make_double2(pr[g], pi[g]);
     __syncthreads();
     if (tid < NS) {
       // coefficient tid = (a, b, c) in the stored order
       int d = 0;
       while ((d + 1)*(d + 1) <= tid) ++d;
       const int o = tid - d*d, a = o > d, b = a ? o - d - 1 : o, c = d - a - b;
-      const int base = a ? M2PPoly<ORD>::N0 : 0;
       double lr = 0, li = 0;
       for (int j = (b + 1)/2; j <= b; ++j)
         for (int l = (c + 1)/2; l <= c; ++l) {
           const int nn = j + l, be = 2*j - b, ga = 2*l - c;
-          const double2 v = sPhi[base + tet(nn) + be*(nn + 1) - be*(be - 1)/2 + ga];
+          const double2 v = sPhi[a*P::NA + sBase[nn] + P::row(nn, be) + ga - P::lo(0, nn, be)];
           const double f = ht[b*HS + j]*ht[c*HS + l];
           lr += f*v.x;
           li += f*v.y;
@@ -831,13 +983,13 @@ extern "C" int sumpyhip_m2p_helmholtz(const sumpyhip_expn *expn, double k, doubl
 #define SUMPY_M2P_POLY(O)                                                                  \
   case O:                                                                                  \
     if (precision)                                                                         \
-      m2p_helm3d_poly<O, float><<<grid, 64, 0, st>>>(                                      \
+      m2p_helm3d_poly<O, float><<<grid, 64*M2PH_NW<float>, 0, st>>>(                       \
           k, ntgt_boxes, target_boxes, source_box_starts, source_box_lists,                \
           box_target_starts, box_target_counts_nonchild, box_centers, nboxes, tx, ty, tz,  \
           rscale, scale, static_cast<const double2 *>(src_expansions), src_base_ibox,      \
           static_cast<double2 *>(pot));                                                    \
     else                                                                                   \
-      m2p_helm3d_poly<O, double><<<grid, 64, 0, st>>>(                                     \
+      m2p_helm3d_poly<O, double><<<grid, 64*M2PH_NW<double>, 0, st>>>(                     \
           k, ntgt_boxes, target_boxes, source_box_starts, source_box_lists,                \
           box_target_starts, box_target_counts_nonchild, box_centers, nboxes, tx, ty, tz,  \
           rscale, scale, static_cast<const double2 *>(src_expansions), src_base_ibox,      \
