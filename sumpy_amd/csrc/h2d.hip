@@ -131,21 +131,20 @@ __device__ __forceinline__ double unit(double vx, double vy, double &ux, double 
   return r;
 }
 
-// Per-lane accumulation of sum_c w Z_c e^{i s c th} over c = -p..p into
-// acc[c + p] (Z: the sequence, c >= 0); the phase e^{i th} is (ux, uy) and
-// s = sign.
-__device__ void add_terms(int p, cplx w, const cplx *Z, double ux, double uy, int sign,
-                          cplx *acc) {
+// put(p + c, w Z_c e^{i s c th}) for c = -p..p (Z: the sequence, c >= 0); the
+// phase e^{i th} is (ux, uy) and s = sign.
+template <class Put>
+__device__ __forceinline__ void add_terms(int p, cplx w, const cplx *Z, double ux, double uy,
+                                          int sign, Put &&put) {
   const cplx e1 = {ux, sign*uy};
   cplx ph = {1.0, 0.0};  // e^{i s c th}
   for (int c = 0; c <= p; ++c) {
     const cplx z = Z[c];
-    const cplx t = cmul(w, cmul(z, ph));
-    acc[p + c] = cadd(acc[p + c], t);
+    put(p + c, cmul(w, cmul(z, ph)));
     if (c > 0) {
       // c -> -c: Z_-c = (-1)^c Z_c, e^{-i s c th} = conj(ph)
       const cplx tn = cmul(w, cmul(z, conj(ph)));
-      acc[p - c] = cadd(acc[p - c], (c & 1) ? cscale(tn, -1.0) : tn);
+      put(p - c, (c & 1) ? cscale(tn, -1.0) : tn);
     }
     ph = cmul(ph, e1);
   }
@@ -157,45 +156,46 @@ __device__ __forceinline__ cplx sarg(cplx kk) {
   return KIND == 1 ? cplx{0.0, kk.re} : kk;
 }
 
-// acc[p + c] += v for |c| <= p
-__device__ __forceinline__ void acc_add(int p, int c, cplx v, cplx *acc) {
-  if (c >= -p && c <= p) acc[p + c] = cadd(acc[p + c], v);
-}
-
 // Derivatives of F_c = Z_c(s r) e^{i sg c th} (sg = +-1) by the shifts
 // W F_c = -s F_{c+1}, Wbar F_c = s F_{c-1} (W = d_x + i d_y):
 //   d_x F_c = (s/2) (F_{c-1} - F_{c+1}),  d_y F_c = (i sg s/2) (F_{c-1} + F_{c+1}),
 // so n . grad F_c = (s/2) ((n_x + i sg n_y) F_{c-1} - (n_x - i sg n_y) F_{c+1}).
-// Per-lane accumulation of w F_c + a F_{c-1} - b F_{c+1} over c = -p..p; Z
-// holds Z_0..Z_{p+1}.  A dipole weight u (contributing u . grad_d G(t - s),
-// i.e. -u . grad_s) gives a = -(s/2)(u_x + i sg u_y), b = -(s/2)(u_x - i sg u_y).
-__device__ void add_terms_der(int p, cplx w, cplx a, cplx b, const cplx *Z, double ux,
-                              double uy, int sign, cplx *acc) {
+// put(p + c, w F_c + a F_{c-1} - b F_{c+1}) for c = -p..p; Z holds Z_0..Z_{p+1}.
+// A dipole weight u (contributing u . grad_d G(t - s), i.e. -u . grad_s) gives
+// a = -(s/2)(u_x + i sg u_y), b = -(s/2)(u_x - i sg u_y).
+template <class Put>
+__device__ __forceinline__ void add_terms_der(int p, cplx w, cplx a, cplx b, const cplx *Z,
+                                              double ux, double uy, int sign, Put &&put) {
   const cplx e1 = {ux, sign*uy};
   const cplx mb = {-b.re, -b.im};
-  cplx ph = {1.0, 0.0};
-  for (int m = 0; m <= p + 1; ++m) {
-    const cplx f = cmul(Z[m], ph);
-    acc_add(p, m, cmul(w, f), acc);
-    acc_add(p, m + 1, cmul(a, f), acc);
-    acc_add(p, m - 1, cmul(mb, f), acc);
-    if (m > 0) {
-      // F_-m = (-1)^m Z_m e^{-i sg m th}
-      cplx fn = cmul(Z[m], conj(ph));
-      if (m & 1) fn = cscale(fn, -1.0);
-      acc_add(p, -m, cmul(w, fn), acc);
-      acc_add(p, -m + 1, cmul(a, fn), acc);
-      acc_add(p, -m - 1, cmul(mb, fn), acc);
-    }
+  cplx ph = e1;
+  // F_{m-1}, F_m, F_{m+1} and F_{-m+1}, F_{-m}, F_{-m-1} with
+  // F_-m = (-1)^m Z_m e^{-i sg m th}
+  cplx f1 = Z[0], f2 = cmul(Z[1], ph), n2 = cscale(cmul(Z[1], conj(ph)), -1.0), f0 = n2,
+       n1 = f1, n0 = f2;
+  for (int m = 0; m <= p; ++m) {
+    put(p + m, cfma(w, f1, cfma(a, f0, cmul(mb, f2))));
+    if (m > 0) put(p - m, cfma(w, n1, cfma(a, n2, cmul(mb, n0))));
+    if (m == p) break;
     ph = cmul(ph, e1);
+    f0 = f1; f1 = f2; f2 = cmul(Z[m + 2], ph);
+    n0 = n1; n1 = n2;
+    n2 = cscale(cmul(Z[m + 2], conj(ph)), (m & 1) ? -1.0 : 1.0);
   }
 }
 
-// {{{ P2M / P2L: one wave per box, lanes over its sources
+// {{{ P2M / P2L: one wave per box (P2L: LW), lanes over its sources
 
-// DER: dipole weights qdx, qdy (either may be null) beside the charges
-template <int KIND, bool LOCAL, bool DER>
-__global__ __launch_bounds__(WAVE) void h2d_p2e_kernel(
+// waves of a target box in the list kernels: few boxes have a list 3 or 4, with
+// tens of boxes each, and a pair is a long serial chain
+constexpr int LW = 4;
+
+// DER: dipole weights qdx, qdy (either may be null) beside the charges.  P2L:
+// the waves take every LW-th list-4 box and their sums are added in order.  A
+// lane's terms are summed over the wave at once: sums of a lane's own would
+// take 1 KB of scratch (P2M of 200000 points at order 20 so: 58 us, this way 33).
+template <int KIND, bool LOCAL, bool DER, int W = LOCAL ? LW : 1>
+__global__ __launch_bounds__(W*WAVE) void h2d_p2e_kernel(
     int p, cplx kk, int nboxes, const int *boxes, const int *starts, const int *lists,
     const int *bss, const int *bsc, const double *centers, int ncenters, const double *sx,
     const double *sy, const double *q, const double *qdx, const double *qdy, double rscale,
@@ -203,18 +203,23 @@ __global__ __launch_bounds__(WAVE) void h2d_p2e_kernel(
   const int ib = blockIdx.x;
   if (ib >= nboxes) return;
   const int box = boxes[ib];
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x % WAVE;
+  const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x/WAVE);
   const double cx = centers[box], cy = centers[ncenters + box];
-  cplx acc[2*PMAX + 1];
-  for (int c = 0; c < 2*p + 1; ++c) acc[c] = {0.0, 0.0};
+  cplx mine = {0.0, 0.0};  // the wave's coefficient of this lane
   cplx Z[PMAX + 2];
   // P2M: the box's own sources; P2L: the sources of its list-4 boxes
   const int e0 = LOCAL ? starts[ib] : 0, e1 = LOCAL ? starts[ib + 1] : 1;
-  for (int e = e0; e < e1; ++e) {
+  for (int e = e0 + wave; e < e1; e += W) {
     const int sb = LOCAL ? lists[e] : box;
     const int s0 = bss[sb], ns = bsc[sb];
-    for (int i = lane; i < ns; i += WAVE) {
-      const int s = s0 + i;
+    for (int i = 0; i < ns; i += WAVE) {
+      const bool active = i + lane < ns;
+      const int s = s0 + (active ? i + lane : 0);
+      auto put = [&](int c, cplx v) {
+        const double re = wave_sum(active ? v.re : 0.0), im = wave_sum(active ? v.im : 0.0);
+        if (lane == c) mine = cadd(mine, cplx{re, im});
+      };
       double ux, uy;  // e^{i th_s}: the source about the centre
       const double rho = unit(sx[s] - cx, sy[s] - cy, ux, uy);
       const cplx w = {q[2*s], q[2*s + 1]};
@@ -227,28 +232,27 @@ __global__ __launch_bounds__(WAVE) void h2d_p2e_kernel(
         const cplx a = cmul(h, cadd(dx, idy)), b = cmul(h, cplx{dx.re - idy.re, dx.im - idy.im});
         if (LOCAL) seq_h<KIND>(kk, rho, p + 1, Z);
         else seq_j<KIND>(kk, rho, p + 1, Z);
-        add_terms_der(p, w, a, b, Z, ux, uy, sg, acc);
+        add_terms_der(p, w, a, b, Z, ux, uy, sg, put);
       } else if (LOCAL) {
         seq_h<KIND>(kk, rho, p > 0 ? p : 1, Z);
-        add_terms(p, w, Z, ux, uy, 1, acc);
+        add_terms(p, w, Z, ux, uy, 1, put);
       } else {
         seq_j<KIND>(kk, rho, p, Z);
-        add_terms(p, w, Z, ux, uy, -1, acc);
+        add_terms(p, w, Z, ux, uy, -1, put);
       }
     }
   }
-  double mine_re = 0.0, mine_im = 0.0;
-  for (int c = 0; c < 2*p + 1; ++c) {
-    const double re = wave_sum(acc[c].re), im = wave_sum(acc[c].im);
-    if (lane == c) {
-      mine_re = re;
-      mine_im = im;
-    }
+  if constexpr (W > 1) {
+    __shared__ cplx part[W][WAVE];
+    part[wave][lane] = mine;
+    __syncthreads();
+    if (wave) return;
+    for (int w = 1; w < W; ++w) mine = cadd(mine, part[w][lane]);
   }
   if (lane < 2*p + 1) {
     const int ac = lane > p ? lane - p : p - lane;
     const double s = LOCAL ? ipow(rscale, ac) : 1.0/ipow(rscale, ac);
-    store_c(out, (long)(box - base)*(2*p + 1) + lane, {mine_re*s, mine_im*s});
+    store_c(out, (long)(box - base)*(2*p + 1) + lane, cscale(mine, s));
   }
 }
 
@@ -256,22 +260,19 @@ __global__ __launch_bounds__(WAVE) void h2d_p2e_kernel(
 
 // {{{ M2M / L2L: one wave per target box
 
-// J_n(s|d|) and e^{i n th_d} for n = 0..N into LDS (lane 0), the same wave
+// J_n(s|d|) and e^{i n th_d} for n = 0..N into LDS (one lane)
 template <int KIND>
 __device__ void shift_data(cplx kk, double dx, double dy, int N, cplx *Js, cplx *ph) {
-  if (threadIdx.x == 0) {
-    double ux, uy;
-    const double dl = unit(dx, dy, ux, uy);
-    cplx Z[NSEQ];
-    seq_j<KIND>(kk, dl, N, Z);
-    cplx e = {1.0, 0.0};
-    for (int n = 0; n <= N; ++n) {
-      Js[n] = Z[n];
-      ph[n] = e;
-      e = cmul(e, cplx{ux, uy});
-    }
+  double ux, uy;
+  const double dl = unit(dx, dy, ux, uy);
+  cplx Z[NSEQ];
+  seq_j<KIND>(kk, dl, N, Z);
+  cplx e = {1.0, 0.0};
+  for (int n = 0; n <= N; ++n) {
+    Js[n] = Z[n];
+    ph[n] = e;
+    e = cmul(e, cplx{ux, uy});
   }
-  __syncthreads();
 }
 
 // J_n e^{i s n th} for any sign of n from the n >= 0 tables (J_-n = (-1)^n J_n)
@@ -284,13 +285,18 @@ __device__ __forceinline__ cplx shift_term(int n, const cplx *Js, const cplx *ph
   return cmul(e, j);
 }
 
+// The Bessel sequences of the relatives, serial chains of 25 us at order 20,
+// run side by side in a lane each (M2M of a level by one lane 90 us, this way
+// 37 us).
 template <int KIND, bool LOCAL>
 __global__ __launch_bounds__(WAVE) void h2d_shift_kernel(
     int ps, int pt, cplx kk, int ntgt, const int *target_boxes, const int *relatives,
     int nboxes, const double *centers, int ncenters, double src_rscale, double tgt_rscale,
     const double *src, int sbase, double *tgt, int tbase) {
-  __shared__ cplx Js[NSEQ];
-  __shared__ cplx ph[NSEQ];
+  // M2M: the (up to 4) children; L2L: the parent
+  constexpr int NREL = LOCAL ? 1 : 4;
+  __shared__ cplx Js[NREL][NSEQ];
+  __shared__ cplx ph[NREL][NSEQ];
   __shared__ cplx S[2*PMAX + 1];
   const int it = blockIdx.x;
   if (it >= ntgt) return;
@@ -298,13 +304,19 @@ __global__ __launch_bounds__(WAVE) void h2d_shift_kernel(
   const int lane = threadIdx.x;
   const int cj = lane - pt;
   cplx acc = {0.0, 0.0};
-  // M2M: the (up to 4) children; L2L: the parent
-  const int nrel = LOCAL ? 1 : 4;
-  for (int r = 0; r < nrel; ++r) {
-    const int sb = LOCAL ? relatives[tb] : relatives[(long)r*nboxes + tb];
+  auto relative = [&](int r) {
+    return LOCAL ? relatives[tb] : relatives[(long)r*nboxes + tb];
+  };
+  if (lane < NREL) {
+    const int sb = relative(lane);
+    if (LOCAL || sb != 0)
+      shift_data<KIND>(kk, centers[tb] - centers[sb],
+                       centers[ncenters + tb] - centers[ncenters + sb], ps + pt, Js[lane],
+                       ph[lane]);
+  }
+  for (int r = 0; r < NREL; ++r) {
+    const int sb = relative(r);
     if (!LOCAL && sb == 0) continue;  // same on every lane
-    const double dx = centers[tb] - centers[sb], dy = centers[ncenters + tb] - centers[ncenters + sb];
-    shift_data<KIND>(kk, dx, dy, ps + pt, Js, ph);
     if (lane < 2*ps + 1) {
       const int am = lane > ps ? lane - ps : ps - lane;
       const double s = LOCAL ? 1.0/ipow(src_rscale, am) : ipow(src_rscale, am);
@@ -313,7 +325,7 @@ __global__ __launch_bounds__(WAVE) void h2d_shift_kernel(
     __syncthreads();
     if (lane < 2*pt + 1)
       for (int mi = 0; mi < 2*ps + 1; ++mi)
-        acc = cfma(S[mi], shift_term(mi - ps - cj, Js, ph, LOCAL ? -1 : 1), acc);
+        acc = cfma(S[mi], shift_term(mi - ps - cj, Js[r], ph[r], LOCAL ? -1 : 1), acc);
     __syncthreads();
   }
   if (lane < 2*pt + 1) {
@@ -420,17 +432,22 @@ __global__ __launch_bounds__(W*WAVE) void h2d_m2l_kernel(
 __device__ __forceinline__ cplx scale_i4(cplx z) { return {-0.25*z.im, 0.25*z.re}; }
 
 // DER: the gradient into gx, gy and the potential into out, any of them null
-template <int KIND, bool MPOLE, bool DER>
-__global__ __launch_bounds__(WAVE) void h2d_e2p_kernel(
+// M2P: LW waves per box, each on every LW-th list-3 box, their sums added in
+// order (429 boxes of 200000 points at order 20: 240 us by one wave each, 66 us
+// by eight; blocks of four find room beside the near field, which eight wait for).
+template <int KIND, bool MPOLE, bool DER, int W = MPOLE ? LW : 1>
+__global__ __launch_bounds__(W*WAVE) void h2d_e2p_kernel(
     int p, cplx kk, int ntgt, const int *target_boxes, const int *starts, const int *lists,
     const int *bts, const int *btc, const double *centers, int ncenters, const double *tx,
     const double *ty, double rscale, const double *coeffs, int base, double *out, double *gx,
     double *gy) {
-  __shared__ cplx S[2*PMAX + 1];
+  __shared__ cplx Sw[W][2*PMAX + 1];
   const int it = blockIdx.x;
   if (it >= ntgt) return;
   const int tb = target_boxes[it];
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x % WAVE;
+  const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x/WAVE);
+  cplx *S = Sw[wave];
   const int t0 = bts[tb], nt = btc[tb];
   const int e0 = MPOLE ? starts[it] : 0, e1 = MPOLE ? starts[it + 1] : 1;
   cplx Z[PMAX + 2];
@@ -438,14 +455,15 @@ __global__ __launch_bounds__(WAVE) void h2d_e2p_kernel(
     const int t = t0 + c0 + lane;
     const bool active = c0 + lane < nt;
     cplx acc = {0.0, 0.0}, accx = {0.0, 0.0}, accy = {0.0, 0.0};
-    for (int e = e0; e < e1; ++e) {
+    for (int e = e0 + wave; e < e1; e += W) {
       const int sb = MPOLE ? lists[e] : tb;
+      wave_sync();  // the previous box's S is read
       if (lane < 2*p + 1) {
         const int ac = lane > p ? lane - p : p - lane;
         const double s = MPOLE ? ipow(rscale, ac) : 1.0/ipow(rscale, ac);
         S[lane] = cscale(load_c(coeffs, (long)(sb - base)*(2*p + 1) + lane), s);
       }
-      __syncthreads();
+      wave_sync();
       if (active) {
         double ux, uy;
         const double rho = unit(tx[t] - centers[sb], ty[t] - centers[ncenters + sb], ux, uy);
@@ -490,9 +508,26 @@ __global__ __launch_bounds__(WAVE) void h2d_e2p_kernel(
         }
         }
       }
+    }
+    if constexpr (W > 1) {
+      __shared__ cplx part[DER ? 3 : 1][W][WAVE];
+      part[0][wave][lane] = acc;
+      if (DER) {
+        part[1][wave][lane] = accx;
+        part[2][wave][lane] = accy;
+      }
+      __syncthreads();
+      if (wave == 0)
+        for (int w = 1; w < W; ++w) {
+          acc = cadd(acc, part[0][w][lane]);
+          if (DER) {
+            accx = cadd(accx, part[1][w][lane]);
+            accy = cadd(accy, part[2][w][lane]);
+          }
+        }
       __syncthreads();
     }
-    if (active) {
+    if (active && wave == 0) {
       // M2P adds to the targets' values; L2P writes them
       auto put = [&](double *o, cplx v) {
         if (o) store_c(o, t, MPOLE ? cadd(load_c(o, t), v) : v);
@@ -512,50 +547,75 @@ __global__ __launch_bounds__(WAVE) void h2d_e2p_kernel(
 
 // {{{ P2P
 
-// J0(x), Y0(x) for 0 < x <= 4 by their power series,
-//   J0 = sum_m (-x^2/4)^m / (m!)^2,
-//   Y0 = (2/pi) ((ln(x/2) + gamma) J0 + sum_{m>=1} (-1)^(m+1) H_m (x^2/4)^m / (m!)^2)
-// with H_m the harmonic numbers; 17 terms reach 1e-19 at x = 4 (against
-// scipy: 8e-16 on (0, 4]); the coefficients fold to constants when unrolled.
-__device__ __forceinline__ void h0_series(double x, double &j0, double &y0) {
-  const double q = 0.25*x*x;
-  double t = 1.0, j = 1.0, s = 0.0, h = 0.0;
-#pragma unroll
+// The coefficients of q^m in J0 and in the sum of Y0 below (H_m/(m!)^2 with the
+// harmonic numbers H_m), signs included
+struct H0Series {
+  double j[18], s[18];
+};
+constexpr H0Series h0_coefficients() {
+  H0Series c{};
+  double f = 1.0, h = 0.0;
+  c.j[0] = 1.0;
   for (int m = 1; m <= 17; ++m) {
-    t *= -q*(1.0/((double)m*(double)m));
+    f *= -1.0/((double)m*(double)m);
     h += 1.0/(double)m;
-    j += t;
-    s -= t*h;
+    c.j[m] = f;
+    c.s[m] = -f*h;
   }
-  j0 = j;
-  y0 = (2.0/PI)*((log(0.5*x) + EULER_GAMMA)*j + s);
+  return c;
 }
 
-// (i/4) H0(k r) for r > 0: the power series up to k r = 4, the Miller /
-// Neumann route above it (complex k: the complex Miller / Neumann route);
-// Yukawa: K0(lam r) / (2 pi)
+// J0(x), Y0(x) for 0 < x <= 4 by their power series in q = x^2/4,
+//   J0 = sum_m (-q)^m / (m!)^2,
+//   Y0 = (2/pi) ((ln(x/2) + gamma) J0 + sum_{m>=1} (-1)^(m+1) H_m q^m / (m!)^2);
+// N terms: 17 reach 1e-19 at x = 4, 10 at x = 1.  By Horner's rule, two
+// operations a term, and ln(x/2) = ln(q)/2, so that no root is taken.
+template <int N>
+__device__ __forceinline__ void h0_series(double q, double &j0, double &y0) {
+  constexpr H0Series c = h0_coefficients();
+  double j = c.j[N], s = c.s[N];
+#pragma unroll
+  for (int m = N - 1; m >= 1; --m) {
+    j = fma(j, q, c.j[m]);
+    s = fma(s, q, c.s[m]);
+  }
+  j0 = fma(j, q, 1.0);
+  y0 = (2.0/PI)*((0.5*log(q) + EULER_GAMMA)*j0 + s*q);
+}
+
+// (i/4) H0(k r) for r > 0, given r^2: the power series up to k r = 4, the
+// Miller / Neumann route above it (complex k: the complex Miller / Neumann
+// route); Yukawa: K0(lam r) / (2 pi)
 template <int KIND>
-__device__ __forceinline__ cplx green(cplx kk, double r) {
+__device__ __forceinline__ cplx green(cplx kk, double r2) {
   if (KIND == 2) {
     cplx J[2], Y[2];
-    bessel_jy_c(cmul(kk, cplx{r, 0.0}), 1, J, Y);
+    bessel_jy_c(cmul(kk, cplx{sqrt(r2), 0.0}), 1, J, Y);
     const cplx h = {J[0].re - Y[0].im, J[0].im + Y[0].re};  // H0 = J0 + i Y0
     return {-0.25*h.im, 0.25*h.re};
   }
-  const double x = kk.re*r;
   if (KIND == 1) {
     double I[2], K[2];
-    bessel_ik(x, 1, I, K);
+    bessel_ik(kk.re*sqrt(r2), 1, I, K);
     return {K[0]/(2.0*PI), 0.0};
   }
+  const double q = 0.25*kk.re*kk.re*r2;
   double j0, y0;
-  if (x <= 4.0) {
-    h0_series(x, j0, y0);
+  if (q <= 0.25 && q > 1e-280) {
+    h0_series<10>(q, j0, y0);
+  } else if (q <= 4.0 && q > 1e-280) {
+    h0_series<17>(q, j0, y0);
   } else {
-    double J[2], Y[2];
-    bessel_jy(x, 1, J, Y);
-    j0 = J[0];
-    y0 = Y[0];
+    const double x = kk.re*sqrt(r2);
+    if (x <= 1.0) {  // k^2 r^2 out of the range of doubles, k r is not
+      j0 = 1.0;
+      y0 = (2.0/PI)*(log(0.5*x) + EULER_GAMMA);
+    } else {
+      double J[2], Y[2];
+      bessel_jy(x, 1, J, Y);
+      j0 = J[0];
+      y0 = Y[0];
+    }
   }
   return {-0.25*y0, 0.25*j0};
 }
@@ -607,10 +667,16 @@ __device__ __forceinline__ void pair_der(cplx kk, double dx, double dy, double r
   gy = cadd(gy, cadd(cscale(cmul(w, gpr), dy), cadd(cscale(k2nd, dy), cmul(gpr, wy))));
 }
 
-// one wave per target box, lanes over its targets; sources of list 1.  DER:
+// W waves per target box, lanes over its targets; sources of list 1, the waves
+// on every W-th source of a box, their sums added in order: the boxes differ in
+// size, and one wave per box leaves the GPU idle while the largest end (200000
+// points in FP64: 856 us, 780 us with four, 572 us with the shorter series
+// above; bound by FP64 arithmetic).  DER:
 // dipole weights qdx, qdy and the gradient outputs gx, gy (any may be null)
+constexpr int P2P_W = 4;
+
 template <int KIND, bool DER>
-__global__ __launch_bounds__(WAVE) void h2d_p2p_csr_kernel(
+__global__ __launch_bounds__(P2P_W*WAVE) void h2d_p2p_csr_kernel(
     cplx kk, int ntgt, const int *target_boxes, const int *starts, const int *lists,
     const int *bss, const int *bsc, const int *bts, const int *btc, const double *tx,
     const double *ty, const double *sx, const double *sy, const double *q, const double *qdx,
@@ -619,29 +685,49 @@ __global__ __launch_bounds__(WAVE) void h2d_p2p_csr_kernel(
   if (it >= ntgt) return;
   const int tb = target_boxes[it];
   const int t0 = bts[tb], nt = btc[tb];
-  for (int i = threadIdx.x; i < nt; i += WAVE) {
-    const int t = t0 + i;
+  const int lane = threadIdx.x % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x/WAVE);
+  __shared__ cplx part[DER ? 3 : 1][P2P_W][WAVE];
+  for (int i0 = 0; i0 < nt; i0 += WAVE) {
+    const bool active = i0 + lane < nt;
+    const int t = t0 + i0 + (active ? lane : 0);
     const double x = tx[t], y = ty[t];
     const int self = t2s ? t2s[t] : -1;
     cplx acc = {0.0, 0.0}, ax = {0.0, 0.0}, ay = {0.0, 0.0};
     for (int e = starts[it]; e < starts[it + 1]; ++e) {
       const int sb = lists[e];
       const int s0 = bss[sb], s1 = s0 + bsc[sb];
-      for (int s = s0; s < s1; ++s) {
+      for (int s = s0 + wave; s < s1; s += P2P_W) {
         const double dx = x - sx[s], dy = y - sy[s];
-        const double r = sqrt(dx*dx + dy*dy);
-        if (r == 0.0 || s == self) continue;
+        const double r2 = dx*dx + dy*dy;
+        if (r2 == 0.0 || s == self) continue;
         if (DER)
-          pair_der<KIND>(kk, dx, dy, r, cplx{q[2*s], q[2*s + 1]},
+          pair_der<KIND>(kk, dx, dy, sqrt(r2), cplx{q[2*s], q[2*s + 1]},
                          qdx ? cplx{qdx[2*s], qdx[2*s + 1]} : cplx{0.0, 0.0},
                          qdy ? cplx{qdy[2*s], qdy[2*s + 1]} : cplx{0.0, 0.0}, acc, ax, ay);
         else
-          acc = cfma(green<KIND>(kk, r), cplx{q[2*s], q[2*s + 1]}, acc);
+          acc = cfma(green<KIND>(kk, r2), cplx{q[2*s], q[2*s + 1]}, acc);
       }
     }
-    if (out) store_c(out, t, acc);
-    if (DER && gx) store_c(gx, t, ax);
-    if (DER && gy) store_c(gy, t, ay);
+    part[0][wave][lane] = acc;
+    if (DER) {
+      part[1][wave][lane] = ax;
+      part[2][wave][lane] = ay;
+    }
+    __syncthreads();
+    if (wave == 0 && active) {
+      for (int w = 1; w < P2P_W; ++w) {
+        acc = cadd(acc, part[0][w][lane]);
+        if (DER) {
+          ax = cadd(ax, part[1][w][lane]);
+          ay = cadd(ay, part[2][w][lane]);
+        }
+      }
+      if (out) store_c(out, t, acc);
+      if (DER && gx) store_c(gx, t, ax);
+      if (DER && gy) store_c(gy, t, ay);
+    }
+    __syncthreads();
   }
 }
 
@@ -657,14 +743,14 @@ __global__ void h2d_p2p_dense_kernel(cplx kk, int nt, const double *tx, const do
   cplx acc = {0.0, 0.0}, ax = {0.0, 0.0}, ay = {0.0, 0.0};
   for (int s = 0; s < ns; ++s) {
     const double dx = x - sx[s], dy = y - sy[s];
-    const double r = sqrt(dx*dx + dy*dy);
-    if (r == 0.0 || s == self) continue;
+    const double r2 = dx*dx + dy*dy;
+    if (r2 == 0.0 || s == self) continue;
     if (DER)
-      pair_der<KIND>(kk, dx, dy, r, cplx{q[2*s], q[2*s + 1]},
+      pair_der<KIND>(kk, dx, dy, sqrt(r2), cplx{q[2*s], q[2*s + 1]},
                      qdx ? cplx{qdx[2*s], qdx[2*s + 1]} : cplx{0.0, 0.0},
                      qdy ? cplx{qdy[2*s], qdy[2*s + 1]} : cplx{0.0, 0.0}, acc, ax, ay);
     else
-      acc = cfma(green<KIND>(kk, r), cplx{q[2*s], q[2*s + 1]}, acc);
+      acc = cfma(green<KIND>(kk, r2), cplx{q[2*s], q[2*s + 1]}, acc);
   }
   if (out) store_c(out, t, acc);
   if (DER && gx) store_c(gx, t, ax);
@@ -747,7 +833,7 @@ extern "C" int sumpyhip_h2d_p2l(int kind, int order, double k, double k_im, int 
   if (ntgt == 0) return SUMPYHIP_OK;
   SUMPY_REQUIRE(weights, "h2d_p2l: null charge weights");
 #define P2L_CALL(KD, DR)                                                                    \
-  h2d_p2e_kernel<KD, true, DR><<<ntgt, WAVE, 0, (hipStream_t)stream>>>(                    \
+  h2d_p2e_kernel<KD, true, DR><<<ntgt, LW*WAVE, 0, (hipStream_t)stream>>>(                 \
       order, kk, ntgt, target_boxes, starts, lists, box_source_starts, box_source_counts,  \
       centers, ncenters, sx, sy, (const double *)weights, (const double *)weights_dx,      \
       (const double *)weights_dy, rscale, (double *)out, base)
@@ -875,7 +961,7 @@ extern "C" int sumpyhip_h2d_m2p(int kind, int order, double k, double k_im, int 
   const cplx kk = {k, k_im};
   if (ntgt == 0) return SUMPYHIP_OK;
 #define M2P_CALL(KD, DR)                                                                    \
-  h2d_e2p_kernel<KD, true, DR><<<ntgt, WAVE, 0, (hipStream_t)stream>>>(                    \
+  h2d_e2p_kernel<KD, true, DR><<<ntgt, LW*WAVE, 0, (hipStream_t)stream>>>(                 \
       order, kk, ntgt, target_boxes, starts, lists, box_target_starts, box_target_counts,  \
       centers, ncenters, tx, ty, rscale, (const double *)mpoles, base, (double *)out,      \
       (double *)out_dx, (double *)out_dy)
@@ -898,7 +984,7 @@ extern "C" int sumpyhip_h2d_p2p_csr(int kind, double k, double k_im, int ntgt,
   if (ntgt == 0) return SUMPYHIP_OK;
   SUMPY_REQUIRE(weights, "h2d_p2p_csr: null charge weights");
 #define CSR_CALL(KD, DR)                                                                    \
-  h2d_p2p_csr_kernel<KD, DR><<<ntgt, WAVE, 0, (hipStream_t)stream>>>(                      \
+  h2d_p2p_csr_kernel<KD, DR><<<ntgt, P2P_W*WAVE, 0, (hipStream_t)stream>>>(                \
       kk, ntgt, target_boxes, starts, lists, box_source_starts, box_source_counts,         \
       box_target_starts, box_target_counts, tx, ty, sx, sy, (const double *)weights,       \
       (const double *)weights_dx, (const double *)weights_dy, t2s, (double *)out,          \
