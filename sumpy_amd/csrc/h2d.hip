@@ -260,19 +260,31 @@ __global__ __launch_bounds__(W*WAVE) void h2d_p2e_kernel(
 
 // {{{ M2M / L2L: one wave per target box
 
-// J_n(s|d|) and e^{i n th_d} for n = 0..N into LDS (one lane)
+// J_n(s r), n = 0..N, into LDS (one lane): KIND 2 into Js, the others' real
+// sequences into A for shift_values
 template <int KIND>
-__device__ void shift_data(cplx kk, double dx, double dy, int N, cplx *Js, cplx *ph) {
-  double ux, uy;
-  const double dl = unit(dx, dy, ux, uy);
-  cplx Z[NSEQ];
-  seq_j<KIND>(kk, dl, N, Z);
-  cplx e = {1.0, 0.0};
-  for (int n = 0; n <= N; ++n) {
-    Js[n] = Z[n];
-    ph[n] = e;
-    e = cmul(e, cplx{ux, uy});
+__device__ __forceinline__ void shift_sequence(cplx kk, double r, int N, double *A, cplx *Js) {
+  if (KIND == 2) bessel_jy_c(cmul(kk, cplx{r, 0.0}), N, Js, nullptr);
+  else if (KIND == 1) bessel_ik(kk.re*r, N, A, nullptr);
+  else bessel_jy(kk.re*r, N, A, nullptr);
+}
+
+// lane n <= N: J_n(s r) and e^{i n th} from the sequence and (ux, uy) = e^{i th}
+template <int KIND>
+__device__ __forceinline__ void shift_values(int n, double ux, double uy, const double *A,
+                                             cplx *Js, cplx *ph) {
+  if (KIND != 2) {
+    const double a = A[n];
+    const int q = KIND == 1 ? n & 3 : 0;  // i^n I_n
+    Js[n] = q == 0 ? cplx{a, 0.0} : q == 1 ? cplx{0.0, a} : q == 2 ? cplx{-a, 0.0}
+                                                                   : cplx{0.0, -a};
   }
+  cplx e = {1.0, 0.0}, b = {ux, uy};
+  for (int m = n; m; m >>= 1) {
+    if (m & 1) e = cmul(e, b);
+    b = cmul(b, b);
+  }
+  ph[n] = e;
 }
 
 // J_n e^{i s n th} for any sign of n from the n >= 0 tables (J_-n = (-1)^n J_n)
@@ -285,9 +297,10 @@ __device__ __forceinline__ cplx shift_term(int n, const cplx *Js, const cplx *ph
   return cmul(e, j);
 }
 
-// The Bessel sequences of the relatives, serial chains of 25 us at order 20,
-// run side by side in a lane each (M2M of a level by one lane 90 us, this way
-// 37 us).
+// The Bessel sequences of the relatives are serial chains: they run side by
+// side in a lane each, in LDS, and the other lanes take what follows from them
+// (in one lane with its arrays in scratch, the latency of each access showed:
+// M2M of a level at order 20 90 us, L2L 30 us; this way 27 and 14 us).
 template <int KIND, bool LOCAL>
 __global__ __launch_bounds__(WAVE) void h2d_shift_kernel(
     int ps, int pt, cplx kk, int ntgt, const int *target_boxes, const int *relatives,
@@ -297,6 +310,7 @@ __global__ __launch_bounds__(WAVE) void h2d_shift_kernel(
   constexpr int NREL = LOCAL ? 1 : 4;
   __shared__ cplx Js[NREL][NSEQ];
   __shared__ cplx ph[NREL][NSEQ];
+  __shared__ double A[KIND == 2 ? 1 : NREL][NSEQ];
   __shared__ cplx S[2*PMAX + 1];
   const int it = blockIdx.x;
   if (it >= ntgt) return;
@@ -307,16 +321,26 @@ __global__ __launch_bounds__(WAVE) void h2d_shift_kernel(
   auto relative = [&](int r) {
     return LOCAL ? relatives[tb] : relatives[(long)r*nboxes + tb];
   };
+  // the shift from relative sb: its length and direction
+  auto shift = [&](int sb, double &ux, double &uy) {
+    return unit(centers[tb] - centers[sb], centers[ncenters + tb] - centers[ncenters + sb], ux,
+                uy);
+  };
   if (lane < NREL) {
     const int sb = relative(lane);
+    double ux, uy;
     if (LOCAL || sb != 0)
-      shift_data<KIND>(kk, centers[tb] - centers[sb],
-                       centers[ncenters + tb] - centers[ncenters + sb], ps + pt, Js[lane],
-                       ph[lane]);
+      shift_sequence<KIND>(kk, shift(sb, ux, uy), ps + pt, A[KIND == 2 ? 0 : lane], Js[lane]);
   }
+  __syncthreads();
   for (int r = 0; r < NREL; ++r) {
     const int sb = relative(r);
     if (!LOCAL && sb == 0) continue;  // same on every lane
+    if (lane <= ps + pt) {
+      double ux, uy;
+      shift(sb, ux, uy);
+      shift_values<KIND>(lane, ux, uy, A[KIND == 2 ? 0 : r], Js[r], ph[r]);
+    }
     if (lane < 2*ps + 1) {
       const int am = lane > ps ? lane - ps : ps - lane;
       const double s = LOCAL ? 1.0/ipow(src_rscale, am) : ipow(src_rscale, am);
