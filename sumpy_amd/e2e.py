@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes
 import weakref
+from functools import cached_property
 
 import numpy as np
 import torch
@@ -58,6 +59,29 @@ class E2EBase:
                 self.tgt_expansion.tables_for(actx.device, k, tgt_rscale))
 
 
+def _rows_of(t, n):
+    """Whether *t* holds rows of *n* coefficients (2D, or all rows in one)."""
+    return t.shape[1] == n if t.dim() == 2 else t.numel() % n == 0
+
+
+def _plain_complex(t, n):
+    """Whether a kernel may read *t* as interleaved complex128 rows of *n*: a
+    lazily conjugated or negated view is contiguous too, but its memory does
+    not hold its values."""
+    return (t.dtype == torch.complex128 and t.is_contiguous()
+            and not (t.is_conj() or t.is_neg()) and _rows_of(t, n))
+
+
+def _check_rows(t, n, dtype):
+    """Refuse coefficients that the kernels would misread or read past."""
+    if t.dtype != dtype:
+        raise TypeError(f"expansions must be {dtype}, got {t.dtype}")
+    if t.is_neg():
+        raise ValueError("expansions must not be a lazily negated view")
+    if not _rows_of(t, n):
+        raise ValueError(f"expansions of shape {tuple(t.shape)}: rows must hold {n} coefficients")
+
+
 class _OctantTranslation(E2EBase):
     """Shared machinery of M2M and L2L: when every child of the level sits at
     one of eight fixed offsets from its parent (an octree), the level's
@@ -73,6 +97,11 @@ class _OctantTranslation(E2EBase):
         self._mats = {}
         #: whether the last call took the octant-matrix (MFMA) path
         self.last_call_used_octant_matrices = False
+
+    @cached_property
+    def _row_sizes(self):
+        """Coefficients of a source and of a target box."""
+        return self.src_expansion.table.nstored, self.tgt_expansion.table.nstored
 
     @staticmethod
     def _host_copy(t):
@@ -113,17 +142,23 @@ class _OctantTranslation(E2EBase):
                 self, actx, kwargs)
         src, tgt = kwargs["src_expansions"], kwargs["tgt_expansions"]
         k = expansion_k(self.tgt_expansion.kernel, kwargs, self.tgt_expansion)
+        n_in, n_out = self._row_sizes
         if not tgt.is_complex():
+            _check_rows(src, n_in, torch.float64)
+            _check_rows(tgt, n_out, torch.float64)
             return self._apply(actx, kwargs, src, tgt, k)
         # complex (Helmholtz) expansions: the translation is real-linear with
-        # real matrices; the octant matrices take both planes as they lie, the
-        # per-box kernels one contiguous plane at a time
-        if max(src.shape[1], tgt.shape[1]) <= MAX_PLANE_COEFFS and src.is_contiguous() and \
-                tgt.is_contiguous() and \
+        # real matrices; the octant matrices take both planes as they lie (only
+        # memory that holds the values in that order), the per-box kernels one
+        # contiguous plane at a time
+        if max(n_in, n_out) <= MAX_PLANE_COEFFS and \
+                _plain_complex(src, n_in) and _plain_complex(tgt, n_out) and \
                 self._apply(actx, kwargs, src, tgt, k, planes=2) is not None:
             return tgt
         sr, si = planes(src)
         tr, ti = planes(tgt)
+        for t, n in ((sr, n_in), (tr, n_out)):
+            _check_rows(t, n, torch.float64)
         self._apply(actx, kwargs, sr, tr, k)
         self._apply(actx, kwargs, si, ti, k)
         set_planes(tgt, tr, ti)

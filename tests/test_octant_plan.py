@@ -14,7 +14,7 @@ from sumpy_amd.array_context import TorchArrayContext
 from sumpy_amd.e2e import GROUP, E2EFromChildren, E2EFromParent, _fragment_order
 from sumpy_amd.expansion.local import LinearPDEConformingVolumeTaylorLocalExpansion
 from sumpy_amd.expansion.multipole import LinearPDEConformingVolumeTaylorMultipoleExpansion
-from sumpy_amd.kernel import LaplaceKernel
+from sumpy_amd.kernel import HelmholtzKernel, LaplaceKernel
 from sumpy_amd.tree import build_tree_and_traversal
 
 
@@ -127,3 +127,49 @@ def test_octant_plan_reproduces_per_box_translation(tree, kind):
         oracle.l2l(order, order, tb, th["box_parent_ids"], th["box_centers"], rs_src, rs_tgt,
                    src, int(lbs[sl]), want, int(lbs[tl]))
     assert rel(got, want) < 1e-13
+
+
+def _octant_operands(op, tree, dtype=torch.complex128):
+    trees, trav = tree
+    n = len(op.src_expansion)
+    return dict(src_expansions=torch.ones((trees.nboxes, n), dtype=dtype), src_base_ibox=0,
+                tgt_expansions=torch.zeros((trees.nboxes, n), dtype=dtype), tgt_base_ibox=0,
+                target_boxes=trav.source_parent_boxes, box_child_ids=trees.box_child_ids,
+                box_parent_ids=trees.box_parent_ids, centers=trees.box_centers,
+                src_rscale=1.0, tgt_rscale=1.0, k=1.0)
+
+
+@pytest.mark.parametrize("cls", [E2EFromChildren, E2EFromParent])
+@pytest.mark.parametrize("octant", [True, False])
+def test_translation_operands_are_checked(tree, cls, octant):
+    """Coefficients that the kernels would misread are refused on the host: a
+    lazily conjugated view (its memory holds the other values), one complex and
+    one real operand, other precisions, rows of another order, a view that is
+    negated on the fly."""
+    knl = HelmholtzKernel(3)
+    mp = LinearPDEConformingVolumeTaylorMultipoleExpansion(knl, 3)
+    lc = LinearPDEConformingVolumeTaylorLocalExpansion(knl, 3)
+    exp = mp if cls is E2EFromChildren else lc
+    op = cls(exp, exp, use_octant_matrices=octant)
+    actx = TorchArrayContext("cpu")
+    good = _octant_operands(op, tree)
+    for name in ("src_expansions", "tgt_expansions"):
+        z = good[name]
+        for bad, error, match in (
+                (z.conj(), RuntimeError, "conjugat"),
+                (z.real.contiguous(), (RuntimeError, TypeError), "view_as_real|float64"),
+                (z.to(torch.complex64), TypeError, "complex64|float32"),
+                (z[:, :-1].contiguous(), ValueError, "16 coefficients"),
+                (torch.cat([z, z], dim=1), ValueError, "16 coefficients")):
+            with pytest.raises(error, match=match):
+                op(actx, **dict(good, **{name: bad}))
+    # the same for a real kernel
+    lap = cls(exp.with_kernel(LaplaceKernel(3)), exp.with_kernel(LaplaceKernel(3)),
+              use_octant_matrices=octant)
+    good = _octant_operands(lap, tree, torch.float64)
+    for name in ("src_expansions", "tgt_expansions"):
+        z = good[name]
+        for bad, error in ((z.float(), TypeError), (z[:, 1:].contiguous(), ValueError),
+                           (torch._neg_view(z), ValueError)):
+            with pytest.raises(error):
+                lap(actx, **dict(good, **{name: bad}))
