@@ -367,6 +367,8 @@ extern "C" int sumpyhip_m2l_fold_pack(int precision, int is_complex, int nboxes,
                                       int kpad, const double *src, const int *kmap,
                                       void *packed, void *stream) {
   SUMPY_REQUIRE(precision == 0 || precision == 1, "m2l_fold_pack: precision %d", precision);
+  SUMPY_REQUIRE(nboxes >= 0 && nstored > 0 && kpad > 0 && kpad % 8 == 0 && kpad >= nstored,
+                "m2l_fold_pack: row of %d coefficients as %d", nstored, kpad);
   if (nboxes == 0) return SUMPYHIP_OK;
   const size_t n = (size_t)nboxes*kpad;
   const int grid = (int)((n + 255)/256 < 16384 ? (n + 255)/256 : 16384);
@@ -394,6 +396,8 @@ extern "C" int sumpyhip_m2l_fold_apply(int precision, int is_complex, int order,
   if (rc) return rc;
   SUMPY_REQUIRE(precision == 0 || precision == 1, "m2l_fold_apply: precision %d", precision);
   SUMPY_REQUIRE(max_wg >= 1 && min_slots >= 1, "m2l_fold_apply: bad launch shape");
+  SUMPY_REQUIRE(nstored == (order + 1)*(order + 1),
+                "m2l_fold_apply: %d coefficients at order %d", nstored, order);
   const unsigned long long row = (unsigned long long)sz[2]*8*(is_complex ? 2 : 1)*
                                  (precision == 0 ? 8 : 4);
   SUMPY_REQUIRE((unsigned long long)nboxes*row < (1ull << 31),

@@ -570,6 +570,10 @@ class M2LPreprocessMultipole(E2EBase):
         nb = int(src.shape[0])
         if out.shape[0] != nb:
             raise ValueError("preprocessed array has the wrong number of boxes")
+        if src.dtype not in (torch.float64, torch.complex128):
+            raise TypeError(f"expansions must be float64 or complex128, got {src.dtype}")
+        if src.is_neg():
+            src = src.resolve_neg()
         if src.is_complex():
             # rows Mr, Mi, -Mi per box (the real embedding of the complex
             # contraction); the packing kernel then sees 3 nb real boxes

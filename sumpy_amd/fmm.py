@@ -527,7 +527,8 @@ class SumpyExpansionWrangler:
         args = (actx, _host(level_start_target_box_nrs), target_boxes, src_box_starts,
                 src_box_lists, mpole_exps)
         folded = m2l_fold.runs(self, *args[1:5])
-        if folded is None or not self._m2l_prefers_folded(folded, args):
+        if folded is None or not m2l_fold.takes(self, mpole_exps) or \
+                not self._m2l_prefers_folded(folded, args):
             return self._m2l_class_matrices(*args)
         return self._m2l_folded(folded, args)
 

@@ -145,6 +145,8 @@ def usable(wrangler, order):
     prec = ti.m2l_translation.precision
     if not (1 <= order <= MAX_ORDER) or prec not in PRECISIONS:
         return False
+    if (np.dtype(wrangler.dtype).kind == "c") != ti.get_base_kernel().is_complex_valued:
+        return False  # the class data have the kernel's planes
     mpole, local = ti.multipole_expansion(order), ti.local_expansion(order)
     n = (order + 1)**2
     if len(local) != n or len(mpole) != n or not (mpole.compressed and local.compressed):
@@ -152,6 +154,17 @@ def usable(wrangler, order):
     planes = 2 if np.dtype(wrangler.dtype).kind == "c" else 1
     row = sizes(order)[2]*8*planes*(8 if prec == "fp64" else 4)
     return wrangler.tree.nboxes*row < 2**31
+
+
+def takes(wrangler, mpole_exps):
+    """Whether the kernels may read *mpole_exps* as the rows of all boxes: the
+    wrangler's dtype, every value in place (no lazily conjugated or negated view,
+    whose memory holds other values)."""
+    m = mpole_exps
+    dtype = torch.complex128 if np.dtype(wrangler.dtype).kind == "c" else torch.float64
+    return (m.dtype == dtype and m.dim() == 1 and m.is_contiguous()
+            and not (m.is_conj() or m.is_neg())
+            and m.numel() == int(wrangler.multipole_expansions_level_starts()[-1]))
 
 
 def runs(wrangler, starts, target_boxes, src_box_starts, src_box_lists):
