@@ -170,8 +170,8 @@ def takes(wrangler, mpole_exps):
 def runs(wrangler, starts, target_boxes, src_box_starts, src_box_lists):
     """[(order, levels)] of the folded M2L of a pass: the runs of consecutive
     levels of one order; None where the pass needs the general contraction
-    (other lists than the traversal's own, not an octree in 3D, other
-    expansions)."""
+    (other lists than the traversal's own or a part of a level's target boxes,
+    not an octree in 3D, other expansions)."""
     trav, tree = wrangler.traversal, wrangler.tree
     if not (wrangler.supports_translation_classes and tree.dimensions == 3
             and wrangler.tree_indep.m2l_translation.use_preprocessing
@@ -182,11 +182,14 @@ def runs(wrangler, starts, target_boxes, src_box_starts, src_box_lists):
                       (src_box_lists, "from_sep_siblings_lists")):
         if ary is not getattr(trav, name, None):
             return None
+    own = trav.host["level_start_target_or_target_parent_box_nrs"]
     classes = wrangler.m2l_translation_class_level_start_box_nrs()
     out = []
     for lev in range(tree.nlevels):
         if starts[lev] == starts[lev + 1] or classes[lev] == classes[lev + 1]:
             continue
+        if starts[lev] != own[lev] or starts[lev + 1] != own[lev + 1]:
+            return None
         order = wrangler.level_orders[lev]
         if not usable(wrangler, order):
             return None

@@ -64,6 +64,30 @@ def test_fold_entry_points_check_row_sizes():
         _capi.call("sumpyhip_m2l_fold_pack", 0, 0, 1, 16, 20, None, None, None, None)
 
 
+def test_folded_m2l_takes_whole_levels():
+    """Levels may be left out; a caller's part of a level's target boxes goes to
+    the class matrices (the plan holds all of them)."""
+    import test_gpu_m2l_fold as t
+    from sumpy_amd.array_context import TorchArrayContext
+    from sumpy_amd.tree import build_tree_and_traversal
+    actx = TorchArrayContext("cpu")
+    tree, trav = build_tree_and_traversal(actx, np.random.default_rng(0).random((3, 3000)),
+                                          None, 20)
+    wr = t._wrangler(actx, trav, ORDER, "fp64", None)
+    lists = (trav.target_or_target_parent_boxes, trav.from_sep_siblings_starts,
+             trav.from_sep_siblings_lists)
+    own = trav.host["level_start_target_or_target_parent_box_nrs"]
+    levels = [lev for _, run in m2l_fold.runs(wr, own, *lists) for lev in run]
+    assert len(levels) >= 2
+    lev = levels[-1]
+    without = np.array(own)
+    without[lev + 1:] = own[lev]
+    assert [lv for _, run in m2l_fold.runs(wr, without, *lists) for lv in run] == levels[:-1]
+    part = np.array(own)
+    part[lev + 1:] -= 1
+    assert m2l_fold.runs(wr, part, *lists) is None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("cplx", [False, True])
 def test_folded_m2l_and_other_arrays(actx, cplx):
