@@ -204,9 +204,18 @@ def _plan(actx, wrangler, levels, ax):
     trav, tree = wrangler.traversal, wrangler.tree
     tcd = wrangler.translation_classes_data
     plans = trav.__dict__.setdefault("_m2l_fold_plans", [])
+    # the arrays that the plan is made from, as they are now: a plan does not
+    # outlive their replacement or a change in place
+    arrays = (trav.target_or_target_parent_boxes, trav.from_sep_siblings_starts,
+              trav.from_sep_siblings_lists, tcd.from_sep_siblings_translation_classes,
+              tree.box_centers, tree.box_levels)
+    versions = [a._version for a in arrays]
     for p in plans:
         if p["tcd"] is tcd and p["key"] == (levels, ax):
-            return p
+            if p["versions"] == versions and all(a is b for a, b in zip(p["arrays"], arrays)):
+                return p
+            plans.remove(p)
+            break
     dev = actx.device
     lst = np.asarray(trav.host["level_start_target_or_target_parent_box_nrs"]).astype(np.int64)
     lev_slot = np.full(tree.nlevels, -1, np.int32)
@@ -222,10 +231,8 @@ def _plan(actx, wrangler, levels, ax):
     def i32(a):
         return torch.from_numpy(np.ascontiguousarray(a, np.int32)).to(dev)
 
-    totp = trav.target_or_target_parent_boxes
-    starts, lists = trav.from_sep_siblings_starts, trav.from_sep_siblings_lists
-    classes = tcd.from_sep_siblings_translation_classes
-    centers, box_levels = tree.box_centers.contiguous(), tree.box_levels
+    totp, starts, lists, classes, centers, box_levels = arrays
+    centers = centers.contiguous()
     code_d = i32(code)
     n = int(totp.numel())
     keys = torch.empty(n, dtype=torch.int32, device=dev)
@@ -251,8 +258,8 @@ def _plan(actx, wrangler, levels, ax):
                actx.stream_handle)
     block_cost = torch.zeros(nb + 1, dtype=torch.int64, device=dev)
     torch.cumsum(bcost, 0, out=block_cost[1:])
-    plan = dict(tcd=tcd, key=(levels, ax), nblocks=nb, maxslots=ms, tile_target=tile_target,
-                src=src, slots=slots, costs=costs, type_end=type_end, block_cost=block_cost,
+    plan = dict(tcd=tcd, key=(levels, ax), arrays=arrays, versions=versions, nblocks=nb,
+                maxslots=ms, tile_target=tile_target, src=src, slots=slots, costs=costs, type_end=type_end, block_cost=block_cost,
                 block_level=i32(np.repeat(np.arange(len(levels)), nblocks)))
     # passes on other streams may use the plan at once
     torch.cuda.current_stream(dev).synchronize()

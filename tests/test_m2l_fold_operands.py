@@ -121,3 +121,32 @@ def test_folded_m2l_and_other_arrays(actx, cplx):
             t._m2l(actx, wr, strided)
         with pytest.raises(TypeError):
             t._m2l(actx, wr, m.float())
+
+
+@pytest.mark.gpu
+def test_folded_m2l_after_a_change_of_the_lists(actx, monkeypatch):
+    """A pair's source box replaced in the traversal's list, in place or by a new
+    array: the plan is made again, the result is the class matrices'."""
+    import test_gpu_m2l_fold as t
+    from sumpy_amd.tree_gpu import build_tree_and_traversal_gpu
+    rng = np.random.default_rng(6)
+    pts = torch.from_numpy(rng.random((3, 3000))).to(actx.device)
+    tree, trav = build_tree_and_traversal_gpu(actx, pts, None, 30)
+    wr = t._wrangler(actx, trav, 5, "fp64", None)
+    m = t._random_mpoles(wr, actx, rng)
+    first = t._m2l(actx, wr, m)
+    last = int(trav.from_sep_siblings_lists[-1])
+    assert len(set(tree.host["box_levels"][last - 2:last + 1])) == 1
+    for change in (lambda v: v[-1:].fill_(last - 1),
+                   lambda v: trav.__dict__["_dev"].__setitem__(
+                       "from_sep_siblings_lists", torch.cat([v[:-1], v[-1:] - 1]))):
+        change(trav.from_sep_siblings_lists)
+        got = t._m2l(actx, wr, m)
+        with monkeypatch.context() as mp:
+            mp.setattr(m2l_fold, "runs", lambda *a: None)
+            want = t._m2l(actx, wr, m)
+        scale = want.abs().max()
+        assert (want - first).abs().max() > 1e-6*scale
+        assert (got - want).abs().max() <= 1e-12*scale
+        first = want
+    assert len(trav.__dict__["_m2l_fold_plans"]) == 1
