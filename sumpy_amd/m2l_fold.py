@@ -25,6 +25,7 @@ import torch
 from sumpy_amd import _capi
 from sumpy_amd.expansion import m2l_device_tables
 from sumpy_amd.profiling import kernel_span
+from sumpy_amd.tools import as_i32
 
 WAVES, TCOL, NVEC = 4, 16, 343  # as in the kernels
 MAX_ORDER, MAX_LEVELS = 12, 32
@@ -231,8 +232,8 @@ def _plan(actx, wrangler, levels, ax):
     def i32(a):
         return torch.from_numpy(np.ascontiguousarray(a, np.int32)).to(dev)
 
-    totp, starts, lists, classes, centers, box_levels = arrays
-    centers = centers.contiguous()
+    totp, starts, lists, classes, box_levels = map(as_i32, (*arrays[:4], arrays[5]))
+    centers = tree.box_centers.contiguous()
     code_d = i32(code)
     n = int(totp.numel())
     keys = torch.empty(n, dtype=torch.int32, device=dev)
@@ -259,7 +260,8 @@ def _plan(actx, wrangler, levels, ax):
     block_cost = torch.zeros(nb + 1, dtype=torch.int64, device=dev)
     torch.cumsum(bcost, 0, out=block_cost[1:])
     plan = dict(tcd=tcd, key=(levels, ax), arrays=arrays, versions=versions, nblocks=nb,
-                maxslots=ms, tile_target=tile_target, src=src, slots=slots, costs=costs, type_end=type_end, block_cost=block_cost,
+                maxslots=ms, tile_target=tile_target, src=src, slots=slots, costs=costs,
+                type_end=type_end, block_cost=block_cost,
                 block_level=i32(np.repeat(np.arange(len(levels)), nblocks)))
     # passes on other streams may use the plan at once
     torch.cuda.current_stream(dev).synchronize()

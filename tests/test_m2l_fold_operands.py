@@ -150,3 +150,27 @@ def test_folded_m2l_after_a_change_of_the_lists(actx, monkeypatch):
         assert (got - want).abs().max() <= 1e-12*scale
         first = want
     assert len(trav.__dict__["_m2l_fold_plans"]) == 1
+
+
+@pytest.mark.gpu
+def test_folded_m2l_with_wide_class_numbers(actx, monkeypatch):
+    """Translation classes handed in as 64-bit integers, as the class matrices
+    take them."""
+    import test_gpu_m2l_fold as t
+    from sumpy_amd.tree import TranslationClassesData
+    from sumpy_amd.tree_gpu import build_tree_and_traversal_gpu
+    rng = np.random.default_rng(7)
+    pts = torch.from_numpy(rng.random((3, 3000))).to(actx.device)
+    _, trav = build_tree_and_traversal_gpu(actx, pts, None, 30)
+    wr = t._wrangler(actx, trav, 5, "fp64", None)
+    own = wr.translation_classes_data
+    wr.translation_classes_data = TranslationClassesData(
+        own.from_sep_siblings_translation_classes.long(),
+        own.from_sep_siblings_translation_class_to_distance_vector,
+        own.from_sep_siblings_translation_classes_level_starts)
+    m = t._random_mpoles(wr, actx, rng)
+    got = t._m2l(actx, wr, m)
+    with monkeypatch.context() as mp:
+        mp.setattr(m2l_fold, "runs", lambda *a: None)
+        want = t._m2l(actx, wr, m)
+    assert (got - want).abs().max() <= 1e-12*want.abs().max()
