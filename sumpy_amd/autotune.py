@@ -17,8 +17,12 @@ tile width and split policy and keeps the fastest, per
      schedule digest)
 
 so that a second run on the same kind of tree reads the choice from disk.
-The cache lives in ``$SUMPY_AMD_CACHE_DIR`` (default ``~/.cache/sumpy_amd``)
-as one JSON file; a missing or unreadable file means "not tuned yet".
+The choice between the class matrices and the folded contraction of an octree
+(:mod:`sumpy_amd.m2l_fold`) is kept the same way
+(:meth:`M2LSplitTuner.prefers_folded`).  The cache lives in
+``$SUMPY_AMD_CACHE_DIR`` (default ``~/.cache/sumpy_amd``) as one JSON file for
+the launch shapes and one for the forms; a missing or unreadable file means "not
+tuned yet".
 """
 
 from __future__ import annotations
@@ -31,6 +35,7 @@ import os
 SPLIT_POLICIES = [(f, m) for f in (1, 2, 4, 8) for m in (6, 12, 24)]
 DEFAULT_POLICY = (4, 12)
 _FILE = "autotune.json"
+_FORM_FILE = "autotune_m2l_form.json"
 
 
 def cache_dir() -> str:
@@ -41,8 +46,8 @@ def cache_dir() -> str:
 class TuneCache:
     """A JSON dictionary on disk, read once and rewritten on every store."""
 
-    def __init__(self, directory=None):
-        self.path = os.path.join(directory or cache_dir(), _FILE)
+    def __init__(self, directory=None, file=_FILE):
+        self.path = os.path.join(directory or cache_dir(), file)
         self._data = None
 
     def _load(self):
@@ -99,19 +104,30 @@ def make_shape_key(kernel, order, precision, arch, digest, version=None):
     return make_key(kernel, order, precision, arch, digest, version) + "|tile_width"
 
 
+def _r2(x):
+    """*x* to two significant digits."""
+    x = int(x)
+    if x < 100:
+        return x
+    return round(x, 2 - len(str(x)))
+
+
+def _digest(shape):
+    return hashlib.sha1(repr(shape).encode()).hexdigest()[:16]
+
+
 def schedule_digest(entries):
     """Digest of the work shape of a batch of levels: tiles, slots and pairs
     per level, rounded to two significant digits so that trees of the same
     kind and size share an entry."""
-    def r2(x):
-        x = int(x)
-        if x < 100:
-            return x
-        s = len(str(x)) - 2
-        return round(x, -s)
-    shape = sorted((r2(e["sched"]["ntiles"]), r2(e["sched"]["nslots"]),
-                    r2(e["sched"]["npairs"])) for e in entries)
-    return hashlib.sha1(repr(shape).encode()).hexdigest()[:16]
+    return _digest(sorted((_r2(e["sched"]["ntiles"]), _r2(e["sched"]["nslots"]),
+                           _r2(e["sched"]["npairs"])) for e in entries))
+
+
+def pass_digest(level_targets, npairs):
+    """The same for a whole pass before any schedule is made: target boxes per
+    level and list-2 pairs."""
+    return _digest(([_r2(n) for n in level_targets], _r2(npairs)))
 
 
 def device_arch(device) -> str:
@@ -129,6 +145,8 @@ class M2LSplitTuner:
 
     def __init__(self, cache=None, repeats=3):
         self.cache = cache if cache is not None else TuneCache()
+        #: choices between the folded form and the class matrices
+        self.form_cache = TuneCache(os.path.dirname(self.cache.path), _FORM_FILE)
         self.repeats = repeats
         self._memo = {}
 
@@ -170,19 +188,45 @@ class M2LSplitTuner:
         return best
 
     def _time(self, actx, entries, pol):
-        import torch
-
         from sumpy_amd.e2e import m2l_apply_levels
+        return self._time_call(actx, lambda: m2l_apply_levels(actx, entries, policy=pol))
+
+    def _time_call(self, actx, run):
+        import torch
         stream = torch.cuda.current_stream(actx.device)
-        m2l_apply_levels(actx, entries, policy=pol)  # warm-up (and LDS limits)
+        run()  # warm-up (plans, schedules, LDS limits)
         start = torch.cuda.Event(enable_timing=True)
         stop = torch.cuda.Event(enable_timing=True)
         start.record(stream)
         for _ in range(self.repeats):
-            m2l_apply_levels(actx, entries, policy=pol)
+            run()
         stop.record(stream)
         stop.synchronize()
         return start.elapsed_time(stop)/self.repeats
+
+    def prefers_folded(self, actx, folded, class_matrices, kernel, orders, precision, digest):
+        """Whether a pass of the M2L runs in *folded* () rather than in
+        *class_matrices* (): timed once per kind of tree (*digest*, of
+        :func:`pass_digest`) like the split policy, so that the next tree of the
+        kind takes the same form and makes no schedule for the other one."""
+        import torch
+        key = make_key(kernel, "-".join(map(str, orders)), precision,
+                       device_arch(actx.device), digest) + "|form"
+        got = self._memo.get(key)
+        if got is None:
+            stored = self.form_cache.get(key)
+            if stored is not None:
+                got = bool(stored["folded"])
+        if got is None:
+            if torch.device(actx.device).type == "cuda" and \
+                    torch.cuda.is_current_stream_capturing():
+                return True  # never time inside a graph capture
+            cm, fo = (self._time_call(actx, run) for run in (class_matrices, folded))
+            got = fo <= cm
+            self.form_cache.put(key, {"folded": got, "folded_ms": round(fo, 4),
+                                      "class_matrices_ms": round(cm, 4)})
+        self._memo[key] = got
+        return got
 
     def choose(self, actx, make_entries, kernel, order, precision):
         """(tile width, split policy) for a batch of levels: *make_entries*
@@ -224,4 +268,4 @@ class M2LSplitTuner:
 
 
 __all__ = ["DEFAULT_POLICY", "M2LSplitTuner", "SPLIT_POLICIES", "TuneCache", "cache_dir",
-           "code_version", "make_key", "make_shape_key", "schedule_digest"]
+           "code_version", "make_key", "make_shape_key", "pass_digest", "schedule_digest"]

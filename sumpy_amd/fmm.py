@@ -541,27 +541,24 @@ class SumpyExpansionWrangler:
         return local_exps
 
     def _m2l_prefers_folded(self, folded, args):
-        """Without autotuning: yes.  With it: whether the folded form is the
-        faster one on this wrangler's first pass (3 runs of each, the class
-        matrices with their tuned split), kept for its later passes."""
-        if not self.tree_indep.autotune:
+        """Without autotuning: yes.  With it: the tuner's choice for this kind of
+        tree (:meth:`sumpy_amd.autotune.M2LSplitTuner.prefers_folded`), timed with
+        the class matrices at their tuned split, looked up once per wrangler."""
+        ti = self.tree_indep
+        if not ti.autotune:
             return True
         got = self._memo.get("m2l_prefers_folded")
         if got is None:
-            if torch.cuda.is_current_stream_capturing():
-                return True  # nothing is timed inside a graph capture
-            times = []
-            for run in (lambda: self._m2l_class_matrices(*args),
-                        lambda: self._m2l_folded(folded, args)):
-                run()  # plans, schedules, the split tuner
-                e0, e1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-                e0.record()
-                for _ in range(3):
-                    run()
-                e1.record()
-                e1.synchronize()
-                times.append(e0.elapsed_time(e1))
-            got = self._memo["m2l_prefers_folded"] = times[1] <= times[0]
+            from sumpy_amd.autotune import pass_digest
+            starts = np.asarray(args[1])
+            digest = pass_digest([starts[lev + 1] - starts[lev] for _, levels in folded
+                                  for lev in levels], args[4].numel())
+            got = ti.m2l_tuner.prefers_folded(
+                args[0], lambda: self._m2l_folded(folded, args),
+                lambda: self._m2l_class_matrices(*args), str(ti.get_base_kernel()),
+                [order for order, _ in folded], ti.m2l_translation.precision, digest)
+            if not torch.cuda.is_current_stream_capturing():
+                self._memo["m2l_prefers_folded"] = got
         return got
 
     def _m2l_class_matrices(self, actx, starts, target_boxes, src_box_starts, src_box_lists,
