@@ -419,6 +419,9 @@ __device__ __forceinline__ void m2p_poly_eval(const typename V2T<T>::type *C, T 
     }
     T gr, gi;
     g(n, gr, gi);
+    // far away (|z|^e > 3e38 for some e <= n) R overflows in FP32 where its
+    // g_n, of r >= |z|, has long vanished: zero then, not 0 inf
+    if (sizeof(T) == 4 && gr == T(0) && gi == T(0)) Rr = Ri = T(0);
     ar += gr*Rr - gi*Ri;
     ai += gr*Ri + gi*Rr;
     __builtin_amdgcn_sched_barrier(0);  // no reads of C far ahead: registers

@@ -103,3 +103,49 @@ def test_helmholtz_list34_forms(actx, order, precision):
                                                for i in lists[lstarts[b]:lstarts[b + 1]]]).astype(int)
         sizes = _term_sizes(mis, centers[:, b:b + 1] - pts[:, ids], 1.5) @ np.abs(q_host[ids])
         assert (np.abs(out["fast"] - out["general"])[b] <= tol*sizes).all()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("order", [6, 11, 12])
+def test_helmholtz_m2p_far_targets(actx, order, precision):
+    """Targets at up to 6000 scales from a small source box (a deep box beside a
+    coarse leaf), where the 12th power of the distance, or its product with the
+    moments of large strengths, leaves the range of FP32 while the terms that it
+    belongs to vanish; a box without multipoles stays zero.  Tolerance as above."""
+    from sumpy_amd import E2PFromCSR
+    from sumpy_amd.expansion.multipole import LinearPDEConformingVolumeTaylorMultipoleExpansion
+    from sumpy_amd.kernel import AxisTargetDerivative, HelmholtzKernel
+    rng = np.random.default_rng(order)
+    knl, k = HelmholtzKernel(3), 1e-3
+    r = np.array([30., 300, 1500, 1700, 3000, 6000])
+    d = rng.standard_normal((3, 4))
+    d[:, 0] = [0, 0, -1]
+    d[:, 1] = [0, 0, 1]
+    pts = (d/np.linalg.norm(d, axis=0))[:, :, None]*r
+    pts = pts.reshape(3, -1)
+    def dev(a):
+        return actx.from_numpy(np.ascontiguousarray(a))
+    mp = LinearPDEConformingVolumeTaylorMultipoleExpansion(knl, order)
+    mis = mp.get_coefficient_identifiers()
+    size = 1/np.array([np.prod(np.arange(1, sum(m) + 1), dtype=float) for m in mis])
+    M = (rng.standard_normal((3, len(mp))) + 1j*rng.standard_normal((3, len(mp))))*size
+    M[0] *= 1e8
+    M[2] = 0
+    one = dev(np.array([0, 0, 0], np.int32))
+    npts = pts.shape[1]
+    for source in range(3):
+        res = []
+        for kernels, prec in (([knl], precision),
+                              ([knl] + [AxisTargetDerivative(i, knl) for i in range(3)], "fp64")):
+            res.append(actx.to_numpy(E2PFromCSR(mp, kernels)(
+                actx, src_expansions=dev(M), src_base_ibox=0, targets=dev(pts),
+                result=[torch.zeros(npts, dtype=torch.complex128, device=actx.device)
+                        for _ in kernels],
+                target_boxes=one[:1], source_box_starts=dev(np.array([0, 1], np.int32)),
+                source_box_lists=dev(np.array([source], np.int32)),
+                box_target_starts=one, centers=dev(np.zeros((3, 3))), rscale=1.0, k=k,
+                box_target_counts_nonchild=dev(np.array([npts, 0, 0], np.int32)),
+                list34_precision=prec)[0]))
+        sizes = np.abs(M[source]) @ _term_sizes(mis, pts, k)
+        u = 2.0**-53 if precision == "fp64" else 2.0**-24
+        assert (np.abs(res[0] - res[1]) <= 4*(200 + 8*order)*u*sizes).all()
