@@ -22,6 +22,8 @@
 // contraction of m2l.hip on the real embedding [Lr; Li] = [Ar -Ai; Ai Ar][Mr; Mi].
 #include "common.h"
 
+#include <cfloat>
+
 namespace sumpyhip {
 namespace {
 
@@ -773,11 +775,20 @@ __global__ __launch_bounds__(256, 4) void p2l_helm3d_moments(
             sQG[g][tid] = mk2<T>(T(w.x*cr - w.y*ci), T(w.x*ci + w.y*cr));
             ar = br; ai = bi; br = cr; bi = ci;
           }
+          // FP32: a power (or x y^b) beyond its range only meets a g_n that is
+          // zero or denormal there; held within the range, the products with it
+          // stay finite
+          const double zlim = 0.5*FLT_MAX, ylim = zlim/fmax(1.0, fabs(x));
           double py = 1, pz = 1;
           #pragma unroll
           for (int e = 0; e <= ORD; ++e) {
-            sY[e][tid] = T(py);
-            sZ[e][tid] = T(pz);
+            if constexpr (sizeof(T) == 4) {
+              sY[e][tid] = T(fmin(fmax(py, -ylim), ylim));
+              sZ[e][tid] = T(fmin(fmax(pz, -zlim), zlim));
+            } else {
+              sY[e][tid] = T(py);
+              sZ[e][tid] = T(pz);
+            }
             py *= y;
             pz *= z;
           }

@@ -149,3 +149,45 @@ def test_helmholtz_m2p_far_targets(actx, order, precision):
         sizes = np.abs(M[source]) @ _term_sizes(mis, pts, k)
         u = 2.0**-53 if precision == "fp64" else 2.0**-24
         assert (np.abs(res[0] - res[1]) <= 4*(200 + 8*order)*u*sizes).all()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("order", [6, 11, 12])
+def test_helmholtz_p2l_far_sources(actx, order, precision):
+    """The transpose: sources at up to 6000 scales from a small target box, whose
+    powers leave the range of FP32.  Tolerance as above; in FP32 relative to the
+    largest coefficient, since g_n loses digits below 1e-38."""
+    from sumpy_amd import P2EFromCSR
+    from sumpy_amd.expansion.local import LinearPDEConformingVolumeTaylorLocalExpansion
+    from sumpy_amd.kernel import AxisSourceDerivative, HelmholtzKernel
+    rng = np.random.default_rng(order)
+    knl, k = HelmholtzKernel(3), 1e-3
+    d = rng.standard_normal((3, 4))
+    d[:, 0] = [0, 0, -1]
+    d[:, 1] = [0, 1, 1]
+    def dev(a):
+        return actx.from_numpy(np.ascontiguousarray(a))
+    lc = LinearPDEConformingVolumeTaylorLocalExpansion(knl, order)
+    mis = lc.get_coefficient_identifiers()
+    zero = dev(np.array([0, 0], np.int32))
+    for r in (30., 300, 1500, 1700, 3000, 6000):
+        pts = d/np.linalg.norm(d, axis=0)*r
+        q_host = rng.standard_normal(4) + 1j*rng.standard_normal(4)
+        q = dev(q_host)
+        out = []
+        for skn, prec in (([knl], precision), ([knl, AxisSourceDerivative(0, knl)], "fp64")):
+            L = torch.zeros((2, len(lc)), dtype=torch.complex128, device=actx.device)
+            P2EFromCSR(lc, kernels=skn, strength_usage=list(range(len(skn))))(
+                actx, sources=dev(pts), strengths=[q, 0*q][:len(skn)], tgt_expansions=L,
+                tgt_base_ibox=0, box_source_starts=zero,
+                box_source_counts_nonchild=dev(np.array([4, 4], np.int32)),
+                list34_precision=prec, target_boxes=zero[:1],
+                source_box_starts=dev(np.array([0, 1], np.int32)),
+                source_box_lists=dev(np.array([1], np.int32)),
+                centers=dev(np.zeros((3, 2))), rscale=1.0, k=k)
+            out.append(actx.to_numpy(L)[0])
+        sizes = _term_sizes(mis, -pts, k) @ np.abs(q_host)
+        u = 2.0**-53 if precision == "fp64" else 2.0**-24
+        if precision == "fp32":
+            sizes = sizes.max()
+        assert (np.abs(out[0] - out[1]) <= 4*(200 + 8*order)*u*sizes).all(), r
