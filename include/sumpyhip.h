@@ -860,10 +860,10 @@ int sumpytree_gpu_colleagues(int dim, int nboxes, int nlevels, const int *level,
 /* Interaction list `which` (1: neighbour leaves, 2: well-separated children of
  * the parent's colleagues, 3: separated smaller boxes per source level, 4:
  * separated coarser leaves) of nb boxes; coll as sumpytree_gpu_colleagues
- * writes it.  counts != NULL: the counting pass (list 3: nlevels counts per
- * box); else the writing pass at starts (list 3: offsets per (level, box)),
- * with the translation slot of each list-2 pair in slots and the level's used
- * slots flagged in used. */
+ * writes it (lists 1 and 4: may be NULL, slower).  counts != NULL: the counting
+ * pass (list 3: nlevels counts per box); else the writing pass at starts (list
+ * 3: offsets per (level, box)), with the translation slot of each list-2 pair
+ * in slots and the level's used slots flagged in used. */
 int sumpytree_gpu_list(int which, int dim, int nboxes, int nlevels, const int *level,
                        const int *ix, const int *child, const int *parent, const int *leaf,
                        const int *level_start, const int *src_cumul, const int *src_nonchild,

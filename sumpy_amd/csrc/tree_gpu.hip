@@ -232,29 +232,42 @@ struct Group {
   }
 };
 
-// colleagues (same-level neighbours) of every box, ascending, -1 padded
+// lane's colleague (same-level neighbour) of box b, ascending, -1 past the last:
+// from coll, or searched by its cell where coll is null (every lane takes part)
+__device__ __forceinline__ int colleague(const TreeView &t, const Group &g, const int *coll,
+                                         int b) {
+  const int ncol = t.dim == 3 ? 26 : 8, ncomb = ncol + 1;
+  if (coll) return g.lane < ncol ? coll[(size_t)b*ncol + g.lane] : -1;
+  int cc = g.lane;
+  bool some = false;
+  int64_t ix[3];
+  for (int d = 0; d < t.dim; ++d) {
+    const int off = cc % 3 - 1;
+    cc /= 3;
+    if (off) some = true;
+    ix[d] = t.ix[(size_t)d*t.nboxes + b] + off;
+  }
+  const int j = some && g.lane < ncomb ? find_box(t, t.level[b], ix) : -1;
+  int rank = 0;
+  for (int k = 0; k < ncomb; ++k) {
+    const int o = __shfl(j, k, GRP);
+    rank += o >= 0 && o < j;
+  }
+  int mine = -1;
+  for (int k = 0; k < ncomb; ++k) {
+    const int o = __shfl(j, k, GRP), r = __shfl(rank, k, GRP);
+    if (o >= 0 && r == g.lane) mine = o;
+  }
+  return mine;
+}
+
+// colleagues of every box, ascending, -1 padded
 __global__ void colleagues_kernel(TreeView t, int *coll) {
   const Group g;
-  const int ncol = t.dim == 3 ? 26 : 8, ncomb = ncol + 1;
+  const int ncol = t.dim == 3 ? 26 : 8;
   for (long i = g.first; i < t.nboxes; i += g.step) {
-    int cc = g.lane;
-    bool some = false;
-    int64_t ix[3];
-    for (int d = 0; d < t.dim; ++d) {
-      const int off = cc % 3 - 1;
-      cc /= 3;
-      if (off) some = true;
-      ix[d] = t.ix[(size_t)d*t.nboxes + i] + off;
-    }
-    const int j = some && g.lane < ncomb ? find_box(t, t.level[i], ix) : -1;
-    int rank = 0;
-    for (int k = 0; k < ncomb; ++k) {
-      const int o = __shfl(j, k, GRP);
-      rank += o >= 0 && o < j;
-    }
-    const int n = __popc(g.ballot(j >= 0));
-    if (j >= 0) coll[(size_t)i*ncol + rank] = j;
-    if (g.lane >= n && g.lane < ncol) coll[(size_t)i*ncol + g.lane] = -1;
+    const int c = colleague(t, g, nullptr, i);
+    if (g.lane < ncol) coll[(size_t)i*ncol + g.lane] = c;
   }
 }
 
@@ -296,7 +309,6 @@ __global__ __launch_bounds__(LTB) void list1_kernel(TreeView t, int nt,
   __shared__ int fills[LTB][MAXLEV + 1];
   int *fill = fills[threadIdx.x];
   const Group g;
-  const int ncol = t.dim == 3 ? 26 : 8;
   for (long it = g.first; it < nt; it += g.step) {
     const int tb = target_boxes[it], lt = t.level[tb];
     const int above = g.ancestors(t, tb, lt);
@@ -304,7 +316,7 @@ __global__ __launch_bounds__(LTB) void list1_kernel(TreeView t, int nt,
     int x = -1;
     for (int l = 0; l <= lt; ++l) {
       const int anc = __shfl(above, l, GRP);
-      x = g.lane < ncol ? coll[(size_t)anc*ncol + g.lane] : -1;
+      x = colleague(t, g, coll, anc);
       if (l == lt) {  // the box itself among its colleagues
         const int r = __popc(g.ballot(x >= 0 && x < tb)), left = __shfl_up(x, 1, GRP);
         x = g.lane < r ? x : g.lane == r ? tb : left;
@@ -408,7 +420,6 @@ __global__ __launch_bounds__(LTB) void list4_kernel(TreeView t, int nb, const in
                                                     const int *coll, int *counts,
                                                     const int *starts, int *out) {
   const Group g;
-  const int ncol = t.dim == 3 ? 26 : 8;
   for (long ib = g.first; ib < nb; ib += g.step) {
     const int b = boxes[ib], lp = t.level[b] - 1;
     int n = counts ? 0 : starts[ib];
@@ -416,7 +427,7 @@ __global__ __launch_bounds__(LTB) void list4_kernel(TreeView t, int nb, const in
       const int p = t.parent[b], above = g.ancestors(t, p, lp);
       for (int l = 0; l <= lp; ++l) {
         const int anc = __shfl(above, l, GRP);
-        const int x = g.lane < ncol ? coll[(size_t)anc*ncol + g.lane] : -1;
+        const int x = colleague(t, g, coll, anc);
         const bool ok = x >= 0 && t.leaf[x] && t.src_nonchild[x] > 0 && adjacent(t, x, p) &&
                         !adjacent(t, x, b);
         const unsigned m = g.ballot(ok);
@@ -522,7 +533,10 @@ extern "C" int sumpytree_gpu_list(int which, int dim, int nboxes, int nlevels,
   SUMPY_REQUIRE(which >= 1 && which <= 4, "tree_gpu: list %d", which);
   SUMPY_REQUIRE(nlevels <= MAXLEV, "tree_gpu: at most 32 levels");
   if (nb == 0) return SUMPYHIP_OK;
-  SUMPY_REQUIRE(coll, "tree_gpu: list %d without the colleagues", which);
+  SUMPY_REQUIRE(coll || which == 1 || which == 4, "tree_gpu: list %d without the colleagues",
+                which);
+  SUMPY_REQUIRE(coll || (ix && prefix && level_start),
+                "tree_gpu: list %d without the colleagues and the boxes' cells", which);
   SUMPY_REQUIRE(counts || (starts && out && (which != 2 || (slots && used))),
                 "tree_gpu: list %d writing pass without its output arrays", which);
   TreeView t = make_view(dim, nboxes, nlevels, level, ix, child, parent, leaf, level_start,

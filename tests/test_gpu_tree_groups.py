@@ -32,3 +32,25 @@ def test_group_lists(actx, dim, n, depth, mpb, targets):
     both = ("pile", src, tgt, mpb, host, gpu)
     test_gpu_tree.test_tree_arrays_equal_host_builder(both)
     test_gpu_tree.test_traversal_arrays_equal_host_builder(both)
+
+
+@pytest.mark.parametrize(("dim", "n", "depth", "mpb"), [
+    (3, 1, 1, 1), (3, 9, 1, 1), (3, 4000, 9, 8), (2, 500, 12, 20)])
+def test_lists_1_and_4_without_the_colleagues(actx, monkeypatch, dim, n, depth, mpb):
+    """A caller of the C entry may pass no colleagues for these two lists."""
+    from sumpy_amd import _capi
+    rng = np.random.default_rng(n + depth)
+    src, tgt = _pile(dim, n, depth, rng), rng.random((dim, n//2 + 1))
+    host = build_tree_and_traversal(actx, src, tgt, mpb)
+    call, without = _capi.call, []
+
+    def no_colleagues(name, *args):
+        if name == "sumpytree_gpu_list" and args[0] in (1, 4):
+            without.append(args[13])
+            args = (*args[:13], None, *args[14:])
+        call(name, *args)
+
+    monkeypatch.setattr(_capi, "call", no_colleagues)
+    gpu = build_tree_and_traversal_gpu(actx, src, tgt, mpb)
+    assert without and all(without)
+    test_gpu_tree.test_traversal_arrays_equal_host_builder(("pile", src, tgt, mpb, host, gpu))
