@@ -13,6 +13,7 @@
 from __future__ import annotations
 
 import ctypes
+import threading
 import weakref
 from functools import cached_property
 
@@ -28,6 +29,8 @@ from sumpy_amd.tools import as_i32, expansion_k, helmholtz_k, planes, set_planes
 TILE = 64  # target boxes per M2L tile by default (the HIP kernel's widest tile)
 TILE_WIDTHS = (64, 32)  # the tile widths the contraction kernels are built for
 MAX_PLANE_COEFFS = 256  # coefficients of a complex octant translation
+MATS_KEPT = 64  # octant matrices an operator keeps for trees to come (two deep trees)
+_MATS_LOCK = threading.Lock()
 GROUP = 16  # target boxes per octant-translation group (matches the HIP kernel)
 MIN_SLOTS_PER_SPLIT = 12
 
@@ -124,14 +127,27 @@ class _OctantTranslation(E2EBase):
             (t.data_ptr(), t.numel(), t._version) for t in (tb_t, *others))
         return per, key
 
-    def _matrices(self, actx, offsets, present, src_rscale, tgt_rscale, k=0.0):
+    def _matrices(self, actx, plan, src_rscale, tgt_rscale, k=0.0):
+        """The level's matrices in fragment order: held with the level's plan,
+        which lives as long as its tree, and for other trees of the same box
+        sizes the newest MATS_KEPT of the operator."""
+        offsets, present = plan["offsets"], plan["present"]
         key = (offsets.tobytes(), present.tobytes(), float(src_rscale), float(tgt_rscale),
                float(k))
-        frag = self._mats.get(key)
+        mats = plan.setdefault("mats", {})
+        frag = mats.get((self, key))
+        if frag is not None:
+            return frag
+        with _MATS_LOCK:
+            frag = self._mats.pop(key, None)
         if frag is None:
             T = self._unit_matrices(actx, offsets, present, src_rscale, tgt_rscale, k)
             frag = _fragment_order(T)
-            self._mats[key] = frag
+        with _MATS_LOCK:
+            self._mats[key] = frag  # the newest
+            while len(self._mats) > MATS_KEPT:
+                del self._mats[next(iter(self._mats))]
+        mats[self, key] = frag
         return frag
 
     def __call__(self, actx, **kwargs):
@@ -185,17 +201,17 @@ class _OctantTranslation(E2EBase):
         return T*torch.from_numpy(present.astype(np.float64)).to(actx.device)[:, None, None]
 
     def _launch_octant(self, actx, plan, frag, src, sbase, tgt, tbase, planes=1):
-        st, tt = self._tables(actx)
-        flops = 2.0*st.table.nstored*tt.table.nstored*plan["npairs"]*planes
+        n_in, n_out = self._row_sizes
+        flops = 2.0*n_in*n_out*plan["npairs"]*planes
         partial = None
         if self.octant_inputs_per_target > 1:
-            partial = torch.empty(plan["ngroups"]*8*GROUP*tt.table.nstored*planes,
+            partial = torch.empty(plan["ngroups"]*8*GROUP*n_out*planes,
                                   dtype=torch.float64, device=tgt.device)
         with kernel_span(self.span_name, flops):
             _capi.call("sumpyhip_octant_translate_planes", planes, plan["ngroups"],
                        _capi.ptr(plan["targets"]), _capi.ptr(plan["inputs"]),
                        _capi.ptr(plan["mask"]), int(plan["items"].shape[0]),
-                       _capi.ptr(plan["items"]), tt.table.nstored, st.table.nstored,
+                       _capi.ptr(plan["items"]), n_out, n_in,
                        _capi.ptr(frag), _capi.ptr(src), int(sbase), _capi.ptr(tgt), int(tbase),
                        _capi.ptr(partial), actx.stream_handle)
         return tgt
@@ -309,8 +325,8 @@ class E2EFromChildren(_OctantTranslation):
                 self.last_call_used_octant_matrices = True
                 if "dev" not in plan:
                     plan["dev"] = _plan_arrays(actx, plan)
-                frag = self._matrices(actx, plan["offsets"], plan["present"],
-                                      kwargs["src_rscale"], kwargs["tgt_rscale"], k)
+                frag = self._matrices(actx, plan, kwargs["src_rscale"],
+                                      kwargs["tgt_rscale"], k)
                 return self._launch_octant(actx, dict(plan["dev"], ngroups=plan["ngroups"],
                                                       npairs=plan["npairs"]),
                                            frag, src, kwargs["src_base_ibox"], tgt,
@@ -392,8 +408,8 @@ class E2EFromParent(_OctantTranslation):
                 self.last_call_used_octant_matrices = True
                 if "dev" not in plan:
                     plan["dev"] = _plan_arrays(actx, plan)
-                frag = self._matrices(actx, plan["offsets"], plan["present"],
-                                      kwargs["src_rscale"], kwargs["tgt_rscale"], k)
+                frag = self._matrices(actx, plan, kwargs["src_rscale"],
+                                      kwargs["tgt_rscale"], k)
                 return self._launch_octant(actx, dict(plan["dev"], ngroups=plan["ngroups"],
                                                       npairs=plan["npairs"]),
                                            frag, src, kwargs["src_base_ibox"], tgt,

@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes
 from functools import lru_cache
+from operator import is_
 
 import numpy as np
 import torch
@@ -185,15 +186,16 @@ def runs(wrangler, starts, target_boxes, src_box_starts, src_box_lists):
             return None
     own = trav.host["level_start_target_or_target_parent_box_nrs"]
     classes = wrangler.m2l_translation_class_level_start_box_nrs()
-    out = []
+    out, ok = [], set()
     for lev in range(tree.nlevels):
         if starts[lev] == starts[lev + 1] or classes[lev] == classes[lev + 1]:
             continue
-        if starts[lev] != own[lev] or starts[lev + 1] != own[lev + 1]:
+        if starts is not own and (starts[lev] != own[lev] or starts[lev + 1] != own[lev + 1]):
             return None
         order = wrangler.level_orders[lev]
-        if not usable(wrangler, order):
+        if order not in ok and not usable(wrangler, order):
             return None
+        ok.add(order)
         if out and out[-1][0] == order and out[-1][1][-1] == lev - 1:
             out[-1][1].append(lev)
         else:
@@ -213,7 +215,7 @@ def _plan(actx, wrangler, levels, ax):
     versions = [a._version for a in arrays]
     for p in plans:
         if p["tcd"] is tcd and p["key"] == (levels, ax):
-            if p["versions"] == versions and all(a is b for a, b in zip(p["arrays"], arrays)):
+            if p["versions"] == versions and all(map(is_, p["arrays"], arrays)):
                 return p
             plans.remove(p)
             break

@@ -173,3 +173,43 @@ def test_translation_operands_are_checked(tree, cls, octant):
                            (torch._neg_view(z), ValueError)):
             with pytest.raises(error):
                 lap(actx, **dict(good, **{name: bad}))
+
+
+def test_translation_matrices_do_not_pile_up(monkeypatch):
+    """A new tree for every step: the matrices of trees that are gone are given
+    back but for the newest of them; a tree's own stay with it, whatever came
+    after, and are not made twice."""
+    import gc
+    import weakref
+    made = []
+
+    def unit_matrices(self, actx, offsets, present, src_rscale, tgt_rscale, k=0.0):
+        T = torch.zeros((8, 4, 4), dtype=torch.float64)
+        made.append(src_rscale)
+        return T
+
+    monkeypatch.setattr(E2EFromChildren, "_unit_matrices", unit_matrices)
+    ex = LinearPDEConformingVolumeTaylorMultipoleExpansion(LaplaceKernel(3), 1)
+    op, actx = E2EFromChildren(ex, ex), TorchArrayContext("cpu")
+    centers = torch.tensor([[0.5, 0.25], [0.5, 0.25], [0.5, 0.25]], dtype=torch.float64)
+    child = torch.zeros((8, 2), dtype=torch.int32)
+    child[0, 0] = 1
+
+    def step(tb, rscale):
+        plan = op._plan(tb, child, centers)
+        return op._matrices(actx, plan, rscale, 2*rscale)
+
+    kept = torch.zeros(1, dtype=torch.int32)
+    first = weakref.ref(step(kept, 1.0))
+    frags = []
+    for i in range(300):
+        tb = torch.zeros(1, dtype=torch.int32)
+        frags.append(weakref.ref(step(tb, 2.0 + i)))
+        assert step(tb, 2.0 + i) is frags[-1]()
+    del tb
+    gc.collect()
+    assert sum(f() is not None for f in frags) <= 64 and frags[-1]() is not None
+    assert step(kept, 1.0) is first() and made.count(1.0) == 1
+    # an equal tree takes the matrices that are left
+    step(torch.zeros(1, dtype=torch.int32), 301.0)
+    assert made.count(301.0) == 1
