@@ -318,6 +318,69 @@ def test_m2m_l2l(actx, lap3d, small_tree, order, octant):
     assert rel(actx.to_numpy(out), ref) < 1e-11
 
 
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize(("compressed", "order"), [
+    (True, 10), (True, 11), (True, 12), (True, 15), (False, 7), (False, 8), (False, 9)])
+def test_octant_matrices_equal_per_box_kernels(actx, small_tree, compressed, order, cplx):
+    """The split form at 121 to 256 coefficients (one or two row blocks a wave, 32
+    or 64 k steps) on both planes of complex expansions, against the per-box
+    kernels.  Both sum n products, whose factors pass about 4 p roundings: within
+    2 n + 8 p of them (in u) of the sum of the products' sizes."""
+    from sumpy_amd import E2EFromChildren, E2EFromParent
+    from sumpy_amd.expansion import local as lmod, multipole as mmod
+    from sumpy_amd.kernel import HelmholtzKernel, LaplaceKernel
+    tree, trav = small_tree
+    th, vh = tree.host, trav.host
+    pre = "LinearPDEConforming" if compressed else ""
+    knl = HelmholtzKernel(3) if cplx else LaplaceKernel(3)
+    kw = {"k": 2.0} if cplx else {}
+    rng = np.random.default_rng(order)
+    lbs = th["level_start_box_nrs"]
+    tl = tree.nlevels - 2
+    sl = tl + 1
+    n_t, n_s = lbs[tl + 1] - lbs[tl], lbs[sl + 1] - lbs[sl]
+    rs_s, rs_t = _rscale(tree, sl, order), _rscale(tree, tl, order)
+    lsp = vh["level_start_source_parent_box_nrs"]
+    lst = vh["level_start_target_or_target_parent_box_nrs"]
+    common = dict(centers=tree.box_centers, **kw)
+    m2m = dict(common, src_base_ibox=int(lbs[sl]), tgt_base_ibox=int(lbs[tl]),
+               target_boxes=dev(actx, vh["source_parent_boxes"][lsp[tl]:lsp[tl + 1]]),
+               box_child_ids=tree.box_child_ids, src_rscale=rs_s, tgt_rscale=rs_t)
+    l2l = dict(common, src_base_ibox=int(lbs[tl]), tgt_base_ibox=int(lbs[sl]),
+               target_boxes=dev(actx, vh["target_or_target_parent_boxes"][lst[sl]:lst[sl + 1]]),
+               box_parent_ids=tree.box_parent_ids, src_rscale=rs_t, tgt_rscale=rs_s)
+    for cls, ex, args, n_in, n_out in (
+            (E2EFromChildren, getattr(mmod, pre + "VolumeTaylorMultipoleExpansion"), m2m, n_s, n_t),
+            (E2EFromParent, getattr(lmod, pre + "VolumeTaylorLocalExpansion"), l2l, n_t, n_s)):
+        e = ex(knl, order)
+        n = len(e)
+        src, tgt0 = rng.standard_normal((n_in, n)), rng.standard_normal((n_out, n))
+        if cplx:
+            src = src + 1j*rng.standard_normal(src.shape)
+            tgt0 = tgt0 + 1j*rng.standard_normal(tgt0.shape)
+        out = {}
+        for octant in (True, False):
+            op = cls(e, e, use_octant_matrices=octant)
+            out[octant] = actx.to_numpy(op(actx, src_expansions=dev(actx, src),
+                                           tgt_expansions=dev(actx, tgt0.copy()), **args))
+            assert op.last_call_used_octant_matrices == octant
+        # the sizes of the products: the matrices' absolute values on those of the inputs
+        op = cls(e, e)
+        unit = op._unit_matrices
+        op._unit_matrices = lambda *a, unit=unit: unit(*a).abs()
+        size = np.zeros((n_out, n))
+        for part in ((src.real, src.imag) if cplx else (src,)):
+            z = np.abs(part).astype(src.dtype)
+            size += np.abs(actx.to_numpy(op(actx, src_expansions=dev(actx, z), **dict(
+                args, tgt_expansions=torch.zeros((n_out, n), dtype=dev(actx, z).dtype,
+                                                 device=actx.device)))))
+        size += np.abs(tgt0)
+        err = np.abs(out[True] - out[False])
+        print(cls.__name__, order, compressed, cplx, (err/size).max()*2.0**53, n)
+        assert (err <= (2*n + 8*order)*2.0**-53*size).all()
+        assert (err < size).all() and np.isfinite(out[True]).all()
+
+
 @pytest.mark.parametrize("order", [2, 5, 10, 12])
 def test_l2p_m2p_p2l(actx, lap3d, small_tree, order):
     from sumpy_amd import E2PFromCSR, E2PFromSingleBox, P2EFromCSR

@@ -440,3 +440,73 @@ def test_fmm_target_point_multiplier_2d(actx, deriv_axes):
     e = np.linalg.norm(p0 - ref)/np.linalg.norm(ref)
     print(f"target point multiplier 2D {deriv_axes}: {e:.2e}")
     assert e < 1e-5
+
+
+@pytest.mark.parametrize("kind", ["lap", "helm"])
+@pytest.mark.parametrize(("compressed", "ps", "pt"), [
+    (True, 10, 10), (True, 12, 12), (True, 1, 12), (False, 6, 6), (False, 9, 9), (False, 9, 7)])
+def test_taylor2d_m2l_classes_over_lists(actx, kind, compressed, ps, pt):
+    """The class form with 32 lanes a target coefficient group (up to 32
+    coefficients) and 64 at list lengths about the 8 or 4 groups of a block,
+    against the form without classes.  Both sum the same products, one with
+    another order of the sources: within (terms + 64) eps of the sum of their
+    sizes, which the class form gives for the sizes of data and multipoles."""
+    from sumpy_amd import (
+        E2EFromCSR,
+        M2LGenerateTranslationClassesDependentData,
+        M2LUsingTranslationClassesDependentData,
+    )
+    knl, mcls, lcls = _classes(kind, compressed)
+    mpole, local = mcls(knl, ps), lcls(knl, pt)
+    kw = {"k": _k(kind)} if kind != "lap" else {}
+    lens = [0, 1, 3, 4, 5, 7, 8, 9, 27]
+    nt, ns = len(lens), 30
+    rng = np.random.default_rng(ps + pt)
+    dev = actx.from_numpy
+    i32 = lambda a: dev(np.asarray(a, np.int32))  # noqa: E731
+    # targets at one of two centres, so that the pairs fall into 2 ns classes
+    ang = rng.uniform(0, 2*np.pi, ns)
+    far = rng.uniform(2, 3.5, ns)*np.array([np.cos(ang), np.sin(ang)])
+    own = np.array([[0.0, 0.25], [0.0, -0.125]])
+    which = np.arange(nt) % 2
+    centers = np.concatenate([own[:, which], far], axis=1)
+    lists = [rng.permutation(ns)[:n] for n in lens]
+    flat = np.concatenate(lists)
+    classes = np.concatenate([w*ns + li for w, li in zip(which, lists)])
+    vecs = (own[:, :, None] - far[:, None, :]).reshape(2, 2*ns)
+    rs = 0.5
+    data = torch.zeros((2*ns, local.m2l_translation.translation_classes_dependent_ndata(
+        local, mpole)), dtype=torch.float64, device=actx.device)
+    M2LGenerateTranslationClassesDependentData(mpole, local)(
+        actx, src_rscale=rs, translation_classes_level_start=0, ntranslation_classes=2*ns,
+        m2l_translation_classes_dependent_data=data,
+        m2l_translation_vectors=dev(np.ascontiguousarray(vecs)), ntranslation_vectors=2*ns, **kw)
+    M = rng.standard_normal((ns, len(mpole)))
+    if kind == "helm":
+        M = M + 1j*rng.standard_normal(M.shape)
+    common = dict(src_base_ibox=nt, tgt_base_ibox=0, target_boxes=i32(np.arange(nt)),
+                  src_box_starts=i32(np.cumsum([0, *lens])), src_box_lists=i32(nt + flat),
+                  centers=dev(np.ascontiguousarray(centers)), src_rscale=rs, tgt_rscale=rs, **kw)
+
+    def run(op, m, **more):
+        out = torch.full((nt, len(local)), 7.0, dtype=torch.from_numpy(M).dtype,
+                         device=actx.device)
+        return actx.to_numpy(op(mpole, local)(
+            actx, src_expansions=dev(m), tgt_expansions=out, **common, **more))
+
+    def with_classes(m, d):
+        return run(M2LUsingTranslationClassesDependentData, m,
+                   m2l_translation_classes_dependent_data=d,
+                   translation_classes_level_start=0,
+                   m2l_translation_classes_lists=i32(classes))
+
+    if kind == "helm":
+        sized = torch.view_as_complex(data.view(2*ns, -1, 2)).abs()
+        sized = torch.stack([sized, torch.zeros_like(sized)], dim=-1).reshape(2*ns, -1)
+    else:
+        sized = data.abs()
+    got, want = with_classes(M, data), run(E2EFromCSR, M)
+    size = np.abs(with_classes(np.abs(M).astype(M.dtype), sized))
+    terms = len(mpole)*np.array(lens)[:, None]
+    assert (np.abs(got - want) <= (terms + 64)*2.0**-52*size).all()
+    assert (got[0] == 0).all() and (size[1:] > 0).all()
