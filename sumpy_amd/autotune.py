@@ -149,6 +149,7 @@ class M2LSplitTuner:
         self.form_cache = TuneCache(os.path.dirname(self.cache.path), _FORM_FILE)
         self.repeats = repeats
         self._memo = {}
+        self._forms = {}
 
     def policy(self, actx, entries, kernel, order, precision):
         import torch
@@ -212,7 +213,7 @@ class M2LSplitTuner:
         import torch
         key = make_key(kernel, "-".join(map(str, orders)), precision,
                        device_arch(actx.device), digest) + "|form"
-        got = self._memo.get(key)
+        got = self._forms.get(key)
         if got is None:
             stored = self.form_cache.get(key)
             if stored is not None:
@@ -225,7 +226,7 @@ class M2LSplitTuner:
             got = fo <= cm
             self.form_cache.put(key, {"folded": got, "folded_ms": round(fo, 4),
                                       "class_matrices_ms": round(cm, 4)})
-        self._memo[key] = got
+        self._forms[key] = got
         return got
 
     def choose(self, actx, make_entries, kernel, order, precision):
