@@ -339,8 +339,9 @@ def apply(actx, wrangler, order, levels, mpole_exps, local_exps):
     wg = min(_max_workgroups(pid, int(cplx), order, str(actx.device)),
              -(-plan["nblocks"]*plan["maxslots"]//MIN_SLOTS))
     partial = torch.empty(2*wg*WAVES*planes*nrb*256, dtype=dt, device=actx.device)
+    # of the dense products that the fold replaces
     flops = 2.0*n*n*planes**2*int(wrangler.traversal.from_sep_siblings_lists.numel())
-    with kernel_span(f"m2l_apply_{prec}", flops):
+    with kernel_span(f"m2l_fold_{prec}", flops):
         _capi.call("sumpyhip_m2l_fold_apply", pid, int(cplx), order, plan["nblocks"],
                    plan["maxslots"], b0, nboxes, n,
                    _capi.ptr(plan["tile_target"]), _capi.ptr(plan["src"]),
