@@ -32,9 +32,12 @@
 // about e^{2 Im(k) r} relative to |H_n|, which limits it to moderate Im(k) r.
 // All kinds: Z_-n = (-1)^n Z_n for Z = J, H.
 //
-// Layout: one wave (64 lanes) per box; lane c + p owns coefficient c
-// (2p+1 <= 63), so the orders go up to 31.  Per-source terms are summed per
-// lane and reduced over the wave with a fixed butterfly (deterministic).
+// Layout: a wave (64 lanes) per box for P2M, M2M, L2L and L2P, several waves of
+// one block for the lists (P2L and M2P 4, M2L with class data 8, the near field
+// 4), each on every n-th entry, their sums added in wave order.  Lane c + p owns
+// coefficient c (2p+1 <= 63), so the orders go up to 31; P2M and P2L add each
+// term of 64 sources over the wave as it is formed, with a fixed butterfly.  All
+// sums are deterministic.
 #include "common.h"
 #include "bessel.h"
 
@@ -193,7 +196,8 @@ constexpr int LW = 4;
 // DER: dipole weights qdx, qdy (either may be null) beside the charges.  P2L:
 // the waves take every LW-th list-4 box and their sums are added in order.  A
 // lane's terms are summed over the wave at once: sums of a lane's own would
-// take 1 KB of scratch (P2M of 200000 points at order 20 so: 58 us, this way 33).
+// take 1 KB of scratch (P2M of 200000 points at order 20 so: 270 us in two
+// launches, this way 127).
 template <int KIND, bool LOCAL, bool DER, int W = LOCAL ? LW : 1>
 __global__ __launch_bounds__(W*WAVE) void h2d_p2e_kernel(
     int p, cplx kk, int nboxes, const int *boxes, const int *starts, const int *lists,
@@ -299,8 +303,9 @@ __device__ __forceinline__ cplx shift_term(int n, const cplx *Js, const cplx *ph
 
 // The Bessel sequences of the relatives are serial chains: they run side by
 // side in a lane each, in LDS, and the other lanes take what follows from them
-// (in one lane with its arrays in scratch, the latency of each access showed:
-// M2M of a level at order 20 90 us, L2L 30 us; this way 27 and 14 us).
+// (in one lane with its arrays in scratch, the latency of each access showed: of
+// 200000 points at order 20, M2M of a level 88-131 us, L2L 28-98; this way 26-29
+// and 13-22, L2L up to 55 where it runs beside the near field).
 template <int KIND, bool LOCAL>
 __global__ __launch_bounds__(WAVE) void h2d_shift_kernel(
     int ps, int pt, cplx kk, int ntgt, const int *target_boxes, const int *relatives,
@@ -457,8 +462,9 @@ __device__ __forceinline__ cplx scale_i4(cplx z) { return {-0.25*z.im, 0.25*z.re
 
 // DER: the gradient into gx, gy and the potential into out, any of them null
 // M2P: LW waves per box, each on every LW-th list-3 box, their sums added in
-// order (429 boxes of 200000 points at order 20: 240 us by one wave each, 66 us
-// by eight; blocks of four find room beside the near field, which eight wait for).
+// order (429 boxes of 200000 points at order 20: 240 us by one wave each, 78 us
+// by four; beside the near field 195 us.  Blocks of eight waves took 66 us but
+// waited for the near field's: 650 us beside it).
 template <int KIND, bool MPOLE, bool DER, int W = MPOLE ? LW : 1>
 __global__ __launch_bounds__(W*WAVE) void h2d_e2p_kernel(
     int p, cplx kk, int ntgt, const int *target_boxes, const int *starts, const int *lists,
@@ -694,8 +700,8 @@ __device__ __forceinline__ void pair_der(cplx kk, double dx, double dy, double r
 // W waves per target box, lanes over its targets; sources of list 1, the waves
 // on every W-th source of a box, their sums added in order: the boxes differ in
 // size, and one wave per box leaves the GPU idle while the largest end (200000
-// points in FP64: 856 us, 780 us with four, 572 us with the shorter series
-// above; bound by FP64 arithmetic).  DER:
+// points in FP64: 856 us, 780 us with four, 575 us with the shorter series
+// above, 526 us without the lists beside it; bound by FP64 arithmetic).  DER:
 // dipole weights qdx, qdy and the gradient outputs gx, gy (any may be null)
 constexpr int P2P_W = 4;
 

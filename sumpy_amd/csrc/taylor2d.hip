@@ -618,7 +618,6 @@ struct Val<1> {
 };
 
 constexpr int MTH = 256;                       // threads per block
-constexpr int TGRID = (2*TPMAX + 1)*(2*TPMAX + 1);
 
 template <int KIND, int G>
 __global__ __launch_bounds__(MTH) void t2_m2l_classes(

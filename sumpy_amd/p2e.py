@@ -157,8 +157,8 @@ class P2EFromCSR(P2EBase):
     level (one launch for all of list 4), each with the rscale of its level,
     and ``tgt_expansions`` holds one row per tree box (``rscale`` is then
     only used for the expansion tables); ``list34_precision="fp32"`` then
-    forms the terms and their sums over 64 sources in FP32 and adds those
-    sums in FP64."""
+    forms the terms and their sums over 64 sources (Helmholtz: 32) in FP32
+    and adds those sums in FP64."""
 
     default_name = "p2e_from_csr"
 
