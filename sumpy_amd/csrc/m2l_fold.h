@@ -235,6 +235,11 @@ struct BufLoad<4> {
 // but the row's and the column's is immediate (complex FP64: the parity
 // classes only; its code would take minutes to compile).
 //
+// In FP32 the transform adds up to three roundings per source; the long sums of a
+// workgroup weigh more, so that the caller keeps its ranges short (their sums are
+// added in FP64): the locals are then no further from FP64 than the class
+// matrices'.
+//
 // Bound: issue of the SIMD.  On gfx950 FP64 and FP32 MFMAs do not overlap with
 // VALU instructions, of other waves either (measured: 8000 FP64 MFMAs 229 us,
 // 128000 additions 507 us, both from two waves of a SIMD 729 us), so the
@@ -485,8 +490,8 @@ void fold_apply_kernel(ApplyArgs a) {
   }
 }
 
-// out rows of the blocks whose slots lie in several workgroups: the sum of
-// their partial accumulators in workgroup order
+// out rows of the blocks whose slots lie in several workgroups: the sum in FP64
+// of their partial accumulators in workgroup order
 template <typename T, bool CX>
 __global__ __launch_bounds__(256) void fold_reduce_kernel(ApplyArgs a, int nrb) {
   constexpr int PL = CX ? 2 : 1;
@@ -507,9 +512,9 @@ __global__ __launch_bounds__(256) void fold_reduce_kernel(ApplyArgs a, int nrb) 
     if (row < 0) continue;
     for (int q = 0; q < PL; ++q) {
       const size_t e = ((size_t)q*nrb + rb)*256 + i*64 + lane;
-      T s = part[((size_t)(2*g0 + 1)*WAVES + wave)*tile + e];
+      double s = part[((size_t)(2*g0 + 1)*WAVES + wave)*tile + e];
       for (long long g = g0 + 1; g <= g1; ++g) s += part[((size_t)(2*g)*WAVES + wave)*tile + e];
-      a.out[((size_t)(tb - a.box0)*a.nstored + row)*PL + q] = (double)s;
+      a.out[((size_t)(tb - a.box0)*a.nstored + row)*PL + q] = s;
     }
   }
 }

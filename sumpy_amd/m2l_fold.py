@@ -31,9 +31,32 @@ from sumpy_amd.tools import as_i32
 WAVES, TCOL, NVEC = 4, 16, 343  # as in the kernels
 MAX_ORDER, MAX_LEVELS = 12, 32
 PRECISIONS = {"fp64": 0, "fp32": 1}
-#: slots a workgroup takes at least (fewer leave the pipeline's start and the
-#: partial sums in the lead)
+
+
+#: cost of the most expensive slot, as in the kernels
+MAX_SLOT_COST = 20
+#: slots (of the most expensive kind) that a workgroup takes at least
 MIN_SLOTS = 4
+
+
+def workgroups(precision, cplx, order, cost, resident):
+    """Workgroups that share slots of *cost* in all: those that the GPU holds at
+    once (*resident*) with MIN_SLOTS each, since fewer leave the pipeline's start
+    and the partial sums in the lead.
+
+    In FP32 up to 6 times as many, of 6 slots (orders up to 7: 8; complex: 2).  A
+    workgroup adds its products up in FP32, the workgroups' sums are added in FP64;
+    with one range for each, locals were up to 2 times (order 3; 1.4 at order 10)
+    as far from FP64 as the class matrices', whose tiles are split too.  This way
+    they are nearer on every level (0.3 to 0.97 times over orders 3-10 and 30000 to
+    700000 uniform, clustered and sphere points; complex 0.4 to 0.97, order 12 up
+    to 1.03).  The M2L of 700000 uniform points took 476 us and takes 509 (order 6),
+    1062 and 1145 (order 10), of 150000 on a sphere, complex, order 12 893 and 1001."""
+    g = min(resident, cost//(MIN_SLOTS*MAX_SLOT_COST))
+    if precision == "fp32":
+        slots = 2 if cplx else 8 if order <= 7 else 6
+        g = max(g, min(6*resident, cost//(slots*MAX_SLOT_COST)))
+    return max(g, 1)
 
 
 @lru_cache(maxsize=None)
@@ -265,8 +288,8 @@ def _plan(actx, wrangler, levels, ax):
                 maxslots=ms, tile_target=tile_target, src=src, slots=slots, costs=costs,
                 type_end=type_end, block_cost=block_cost,
                 block_level=i32(np.repeat(np.arange(len(levels)), nblocks)))
-    # passes on other streams may use the plan at once
-    torch.cuda.current_stream(dev).synchronize()
+    # (waits for the plan: passes on other streams may use it at once)
+    plan["cost"] = int(block_cost[-1])
     plans.append(plan)
     return plan
 
@@ -336,8 +359,8 @@ def apply(actx, wrangler, order, levels, mpole_exps, local_exps):
     packed = torch.empty(nboxes*nkp*8*planes, dtype=dt, device=actx.device)
     _capi.call("sumpyhip_m2l_fold_pack", pid, int(cplx), nboxes, n, nkp*8, _capi.ptr(msrc),
                _capi.ptr(kmap), _capi.ptr(packed), actx.stream_handle)
-    wg = min(_max_workgroups(pid, int(cplx), order, str(actx.device)),
-             -(-plan["nblocks"]*plan["maxslots"]//MIN_SLOTS))
+    wg = workgroups(prec, cplx, order, plan["cost"],
+                    _max_workgroups(pid, int(cplx), order, str(actx.device)))
     partial = torch.empty(2*wg*WAVES*planes*nrb*256, dtype=dt, device=actx.device)
     # of the dense products that the fold replaces
     flops = 2.0*n*n*planes**2*int(wrangler.traversal.from_sep_siblings_lists.numel())
@@ -349,7 +372,7 @@ def apply(actx, wrangler, order, levels, mpole_exps, local_exps):
                    _capi.ptr(plan["type_end"]), _capi.ptr(plan["block_level"]),
                    _capi.ptr(plan["block_cost"]), _capi.ptr(row), _capi.ptr(off_t),
                    _capi.ptr(off_s), _capi.ptr(packed), _capi.ptr(table), stride, wg,
-                   MIN_SLOTS, _capi.ptr(partial), _capi.ptr(lout), actx.stream_handle)
+                   1, _capi.ptr(partial), _capi.ptr(lout), actx.stream_handle)
 
 
 __all__ = ["apply", "runs"]

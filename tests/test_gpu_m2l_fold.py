@@ -147,3 +147,37 @@ def test_folded_m2l_orders_by_level_and_other_lists(actx, monkeypatch):
         trav.from_sep_siblings_lists.clone(), mpoles)
     scale = copied.abs().max()
     assert (got - copied).abs().max() <= 1e-12*scale
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(("kind", "points", "n", "order"), [
+    ("laplace", "uniform", 700_000, 3), ("laplace", "uniform", 700_000, 10),
+    ("laplace", "gaussian", 200_000, 7), ("helmholtz", "sphere", 60_000, 8)])
+def test_folded_fp32_error_is_the_class_matrices(actx, monkeypatch, kind, points, n, order):
+    """In FP32 the folded form is no further from FP64 than the class matrices, on
+    the locals of the points' own multipoles, level by level: the rms over boxes
+    and coefficients relative to the coefficient's rms, whose own scatter between
+    point sets is some percent."""
+    from sumpy_amd.tree_gpu import build_tree_and_traversal_gpu
+    rng = np.random.default_rng(order)
+    pts = torch.from_numpy(_points(points, n, rng)).to(actx.device)
+    tree, trav = build_tree_and_traversal_gpu(actx, pts, None, 64)
+    k = 4.0 if kind == "helmholtz" else None
+    wr64, wr32 = (_wrangler(actx, trav, order, p, k) for p in ("fp64", "fp32"))
+    q = rng.standard_normal(n)
+    q = actx.from_numpy(q + 1j*rng.standard_normal(n) if k else q)
+    h = trav.host
+    m = wr64.form_multipoles(actx, h["level_start_source_box_nrs"], trav.source_boxes, [q])
+    m = wr64.coarsen_multipoles(actx, h["level_start_source_parent_box_nrs"],
+                                trav.source_parent_boxes, m)
+    ref, folded = _m2l(actx, wr64, m), _m2l(actx, wr32, m)
+    monkeypatch.setattr(m2l_fold, "runs", lambda *a: None)
+    matrices = _m2l(actx, wr32, m)
+    for lev in range(2, tree.nlevels):
+        want = wr64.local_expansions_view(ref, lev)[1]
+        size = want.abs().pow(2).mean(0).sqrt()
+        if (size == 0).any():
+            continue
+        err = [float(((wr64.local_expansions_view(x, lev)[1] - want).abs()/size).pow(2)
+                     .mean().sqrt()) for x in (folded, matrices)]
+        assert err[0] <= 1.05*err[1], (lev, err)
