@@ -17,6 +17,7 @@ from.
 from __future__ import annotations
 
 import ctypes
+import math
 from functools import lru_cache
 from operator import is_
 
@@ -44,18 +45,22 @@ def workgroups(precision, cplx, order, cost, resident):
     once (*resident*) with MIN_SLOTS each, since fewer leave the pipeline's start
     and the partial sums in the lead.
 
-    In FP32 up to 6 times as many, of 6 slots (orders up to 7: 8; complex: 2).  A
-    workgroup adds its products up in FP32, the workgroups' sums are added in FP64;
-    with one range for each, locals were up to 2 times (order 3; 1.4 at order 10)
-    as far from FP64 as the class matrices', whose tiles are split too.  This way
-    they are nearer on every level (0.3 to 0.97 times over orders 3-10 and 30000 to
-    700000 uniform, clustered and sphere points; complex 0.4 to 0.97, order 12 up
-    to 1.03).  The M2L of 700000 uniform points took 476 us and takes 509 (order 6),
-    1062 and 1145 (order 10), of 150000 on a sphere, complex, order 12 893 and 1001."""
+    In FP32 up to 6 times as many, of about 6 slots (orders up to 7: 8; complex: 2),
+    in whole rounds: 1.5 rounds of 512 take 1165 us where 2 take 901.  A workgroup
+    adds its products up in FP32, the workgroups' sums are added in FP64; with one
+    range for each, locals were up to 2 times (order 3; 1.4 at order 10) as far from
+    FP64 as the class matrices', whose tiles are split too.  This way they are nearer
+    on all but single levels (0.3 to 1.04 times over orders 3-10 and 30000 to 700000
+    uniform, clustered and sphere points; complex 0.4 to 1.00, order 12 up to 1.03).
+    The M2L of 700000 uniform points took 473 us and takes 502 (order 6), 1067 and
+    1118 (order 10), of 150000 on a sphere, complex, order 12 904 and 953."""
     g = min(resident, cost//(MIN_SLOTS*MAX_SLOT_COST))
     if precision == "fp32":
         slots = 2 if cplx else 8 if order <= 7 else 6
-        g = max(g, min(6*resident, cost//(slots*MAX_SLOT_COST)))
+        more = cost//(slots*MAX_SLOT_COST)
+        if more > resident:  # (a seventh of a round is not worth a whole one)
+            more = min(6, max(1, math.ceil(more/resident - 1/7)))*resident
+        g = max(g, more)
     return max(g, 1)
 
 

@@ -174,3 +174,19 @@ def test_folded_m2l_with_wide_class_numbers(actx, monkeypatch):
         mp.setattr(m2l_fold, "runs", lambda *a: None)
         want = t._m2l(actx, wr, m)
     assert (got - want).abs().max() <= 1e-12*want.abs().max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_workgroups_leave_a_slot_for_each(precision, cplx):
+    """A workgroup's share of the cost is more than the most expensive slot, so that
+    one begins in it (its partial sums are read); whole rounds past the first."""
+    for order in (3, 8, 12):
+        for resident in (1, 256, 768, 2048):
+            for cost in [*range(0, 400, 7), 10**4, 123_457, 10**6, 10**9]:
+                g = m2l_fold.workgroups(precision, cplx, order, cost, resident)
+                assert 1 <= g <= 6*resident
+                assert g == 1 or cost//g > m2l_fold.MAX_SLOT_COST
+                assert g <= resident or g % resident == 0
+                if precision == "fp64":
+                    assert g == max(1, min(resident, cost//80))
